@@ -229,6 +229,9 @@ static std::vector<double> build_tables(const double *f_in, int n)
         T(TB_A0M, j) = k.a0m; T(TB_A1M, j) = k.a1m; T(TB_A2M, j) = k.a2m; T(TB_A3M, j) = k.a3m;
         T(TB_A0P, j) = k.a0p; T(TB_A1P, j) = k.a1p; T(TB_A2P, j) = k.a2p; T(TB_A3P, j) = k.a3p;
     }
+    // the face below cell 0, which the sweeps form as the high face of cell -1: the same
+    // coefficients (ppm_coef takes the four widths around a face by the same expressions)
+    for (int r = 0; r < 4; r++) T(TB_A0P + r, -1) = T(TB_A0M + r, 0);
     return t;
 }
 

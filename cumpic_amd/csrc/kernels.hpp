@@ -140,18 +140,20 @@ template <typename R, int RECON>
 __device__ inline void recon_lane(const Tabs &tb, int ax, int jc, R c, R &vm, R &vp)
 {
     R cm1 = lane_up(c);
-    R cp1 = lane_down(c);
-    if (RECON == 5) {
-        weno5_edges<R>(__shfl_up(c, 2, 64), cm1, c, cp1, __shfl_down(c, 2, 64), vm, vp);
-    } else if (RECON == 4) {
-        R dm = ppm_slope<R>(tb.atr<R>(ax, TB_B0C, jc), tb.atr<R>(ax, TB_B1C, jc), cm1, c, cp1);
-        R dmm1 = lane_up(dm);
-        R dmp1 = lane_down(dm);
-        ppm_edges<R>(tb.atr<R>(ax, TB_A0M, jc), tb.atr<R>(ax, TB_A1M, jc), tb.atr<R>(ax, TB_A2M, jc),
-                     tb.atr<R>(ax, TB_A3M, jc), tb.atr<R>(ax, TB_A0P, jc), tb.atr<R>(ax, TB_A1P, jc),
-                     tb.atr<R>(ax, TB_A2P, jc), tb.atr<R>(ax, TB_A3P, jc), cm1, c, cp1, dmm1, dm, dmp1, vm, vp);
+    if constexpr (RECON == 4) {
+        // each lane forms the difference to its lower neighbour, its limited slope and the value
+        // on its high face; the neighbours' come by lane moves
+        const R dl = c - cm1, dr = lane_down(dl);
+        const R dm = ppm_slope_d<R>(tb.atr<R>(ax, TB_B0C, jc), tb.atr<R>(ax, TB_B1C, jc), dl, dr);
+        const R vr = ppm_face<R>(tb.atr<R>(ax, TB_A0P, jc), tb.atr<R>(ax, TB_A1P, jc), tb.atr<R>(ax, TB_A2P, jc),
+                                 tb.atr<R>(ax, TB_A3P, jc), c, dr, lane_down(dm), dm);
+        ppm_limit<R>(lane_up(vr), vr, c, vm, vp);
     } else {
-        tvd_any<R, RECON>(tb.atr<R>(ax, TB_CF, jc), tb.atr<R>(ax, TB_CB, jc), cm1, c, cp1, vm, vp);
+        R cp1 = lane_down(c);
+        if constexpr (RECON == 5)
+            weno5_edges<R>(__shfl_up(c, 2, 64), cm1, c, cp1, __shfl_down(c, 2, 64), vm, vp);
+        else
+            tvd_any<R, RECON>(tb.atr<R>(ax, TB_CF, jc), tb.atr<R>(ax, TB_CB, jc), cm1, c, cp1, vm, vp);
     }
 }
 
@@ -298,9 +300,10 @@ __device__ inline void flux_ylane_tile(const Lay &L, const Fields<R> &F, const T
 
 
 // ------------------------------------------------------------------------------------------
-// y and z sweeps: each thread walks one pencil along the sweep axis, lanes along x, keeping the
-// 4-cell value window and 3 limited slopes of every reconstructed variable in registers so that
-// each slope, each PPM call and each Riemann solve is computed exactly once.
+// y and z sweeps: each thread walks one pencil along the sweep axis, lanes along x, keeping a
+// sliding window of every reconstructed variable in registers (PPM: two cell values, one limited
+// slope, the low face's value and the lower cell's high edge) so that each slope, each face value,
+// each limiter call and each Riemann solve is computed exactly once.
 // (solver/spatial.f90:474-511 and :552-589)
 // ------------------------------------------------------------------------------------------
 // One 128-thread tile: bx covers px*(nt+2) pencils, segment by of seglen faces along DIR.
@@ -357,7 +360,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
                 const R bn = ldi(sweep_p(F) + ibn * ps, gf);
                 FaceState<R> sl{vp[0], vp[3], vp[1], vp[2], vp[4], bn, vp[5], vp[6]};
                 FaceState<R> sr{vm[0], vm[3], vm[1], vm[2], vm[4], bn, vm[5], vm[6]};
-                riemann_face<3, R, SOLVER>(R(M.ggas), sl, sr, fl);
+                riemann_face<3, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
                 R *o = F.F[2];
                 sti(o, gf, fl[0]);
                 sti(o + 1 * ps, gf, fl[2]);
@@ -370,47 +373,57 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
             }
         }
     }
-    // window: w0 = v(c-1), w1 = v(c), w2 = v(c+1), w3 = v(c+2) ; slopes d0 = dm(c-1), d1 = dm(c), d2 = dm(c+1)
-    R w0[7], w1[7], w2[7], w3[7], d0[7], d1[7], vpp[7];
-    R wm[RECON == 5 ? 7 : 1];  // WENO5: the value two cells back
+    // window: w1 = v(c), w2 = v(c+1), w3 = v(c+2); PPM: d1 = limited slope of c, fl0 = value on the
+    // low face of c; TVD and WENO5: w0 = v(c-1), and for WENO5 wm = v(c-2)
+    R w1[7], w2[7], w3[7], vpp[7];
+    R d1[RECON == 4 ? 7 : 1], fl0[RECON == 4 ? 7 : 1], w0[RECON == 4 ? 1 : 7], wm[RECON == 5 ? 7 : 1];
     {
         R a[7];
         load7(s0 - 2, a);
-        load7(s0 - 1, w0);
-        load7(s0, w1);
-        load7(s0 + 1, w2);
-        if (RECON == 5) {
-#pragma unroll
-            for (int v = 0; v < 7; v++) wm[v] = a[v];
-        }
-        if (RECON == 4) {
+        if constexpr (RECON != 4) load7(s0 - 1, w0);
+        if constexpr (RECON == 4) {
+            R b[7];
+            load7(s0 - 1, b);
+            load7(s0, w1);
+            load7(s0 + 1, w2);
             R b0 = tb.atr<R>(ax, TB_B0C, s0 - 1), b1 = tb.atr<R>(ax, TB_B1C, s0 - 1);
             R c0 = tb.atr<R>(ax, TB_B0C, s0), c1 = tb.atr<R>(ax, TB_B1C, s0);
+            R a0 = tb.atr<R>(ax, TB_A0P, s0 - 1), a1 = tb.atr<R>(ax, TB_A1P, s0 - 1);
+            R a2 = tb.atr<R>(ax, TB_A2P, s0 - 1), a3 = tb.atr<R>(ax, TB_A3P, s0 - 1);
 #pragma unroll
             for (int v = 0; v < 7; v++) {
-                d0[v] = ppm_slope<R>(b0, b1, a[v], w0[v], w1[v]);
-                d1[v] = ppm_slope<R>(c0, c1, w0[v], w1[v], w2[v]);
+                const R d = w1[v] - b[v];
+                const R d0 = ppm_slope_d<R>(b0, b1, b[v] - a[v], d);
+                d1[v] = ppm_slope_d<R>(c0, c1, d, w2[v] - w1[v]);
+                fl0[v] = ppm_face<R>(a0, a1, a2, a3, b[v], d, d1[v], d0);
+            }
+        } else {
+            load7(s0, w1);
+            load7(s0 + 1, w2);
+            if constexpr (RECON == 5) {
+#pragma unroll
+                for (int v = 0; v < 7; v++) wm[v] = a[v];
             }
         }
     }
     for (int c = s0; c <= s1 + 1; c++) {
         load7(c + 2, w3);
         R vm[7], vp[7];
-        if (RECON == 5) {
+        if constexpr (RECON == 5) {
 #pragma unroll
             for (int v = 0; v < 7; v++) weno5_edges<R>(wm[v], w0[v], w1[v], w2[v], w3[v], vm[v], vp[v]);
             weno_positivity<R>(w1, vm, vp);
-        } else if (RECON == 4) {
+        } else if constexpr (RECON == 4) {
             R b0 = tb.atr<R>(ax, TB_B0C, c + 1), b1 = tb.atr<R>(ax, TB_B1C, c + 1);
-            R a0m = tb.atr<R>(ax, TB_A0M, c), a1m = tb.atr<R>(ax, TB_A1M, c), a2m = tb.atr<R>(ax, TB_A2M, c);
-            R a3m = tb.atr<R>(ax, TB_A3M, c), a0p = tb.atr<R>(ax, TB_A0P, c), a1p = tb.atr<R>(ax, TB_A1P, c);
-            R a2p = tb.atr<R>(ax, TB_A2P, c), a3p = tb.atr<R>(ax, TB_A3P, c);
+            R a0 = tb.atr<R>(ax, TB_A0P, c), a1 = tb.atr<R>(ax, TB_A1P, c);
+            R a2 = tb.atr<R>(ax, TB_A2P, c), a3 = tb.atr<R>(ax, TB_A3P, c);
 #pragma unroll
             for (int v = 0; v < 7; v++) {
-                R d2 = ppm_slope<R>(b0, b1, w1[v], w2[v], w3[v]);
-                ppm_edges<R>(a0m, a1m, a2m, a3m, a0p, a1p, a2p, a3p, w0[v], w1[v], w2[v], d0[v], d1[v], d2,
-                             vm[v], vp[v]);
-                d0[v] = d1[v];
+                const R d = w2[v] - w1[v];
+                const R d2 = ppm_slope_d<R>(b0, b1, d, w3[v] - w2[v]);
+                const R vr = ppm_face<R>(a0, a1, a2, a3, w1[v], d, d2, d1[v]);
+                ppm_limit<R>(fl0[v], vr, w1[v], vm[v], vp[v]);
+                fl0[v] = vr;
                 d1[v] = d2;
             }
         } else {
@@ -427,7 +440,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
                 // rotated frame n=y, t1=z, t2=x ; reconstructed cell B order (x, z)
                 FaceState<R> sl{vpp[0], vpp[2], vpp[3], vpp[1], vpp[4], bn, vpp[6], vpp[5]};
                 FaceState<R> sr{vm[0], vm[2], vm[3], vm[1], vm[4], bn, vm[6], vm[5]};
-                riemann_face<2, R, SOLVER>(R(M.ggas), sl, sr, fl);
+                riemann_face<2, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
                 R *o = F.F[1];
                 sti(o, gf, fl[0]);
                 sti(o + 1 * ps, gf, fl[3]);
@@ -440,7 +453,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
                 // rotated frame n=z, t1=x, t2=y ; reconstructed cell B order (x, y)
                 FaceState<R> sl{vpp[0], vpp[3], vpp[1], vpp[2], vpp[4], bn, vpp[5], vpp[6]};
                 FaceState<R> sr{vm[0], vm[3], vm[1], vm[2], vm[4], bn, vm[5], vm[6]};
-                riemann_face<3, R, SOLVER>(R(M.ggas), sl, sr, fl);
+                riemann_face<3, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
                 R *o = F.F[2];
                 sti(o, gf, fl[0]);
                 sti(o + 1 * ps, gf, fl[2]);
@@ -453,9 +466,9 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
         }
 #pragma unroll
         for (int v = 0; v < 7; v++) {
-            if (RECON == 5) wm[v] = w0[v];
+            if constexpr (RECON == 5) wm[v] = w0[v];
+            if constexpr (RECON != 4) w0[v] = w1[v];
             vpp[v] = vp[v];
-            w0[v] = w1[v];
             w1[v] = w2[v];
             w2[v] = w3[v];
         }
