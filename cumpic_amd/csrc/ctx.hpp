@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -158,6 +159,65 @@ void batch_after_run(cumc_batch *b, int nsteps);
 void launch_ghost(cumc_ctx *ctx);
 void launch_ghost32(cumc_ctx *ctx);
 
+// ------------------------------------------------------------------------------------------
+// Segment length of the pencil walks.  A walk of sl faces takes about sl + 1.3 face times (warm-up
+// slopes and face value, first loads), so long segments waste least; but the whole launch lasts as
+// long as its fullest compute unit, so a grid that gives few wavefronts wants short segments.
+// The load of a compute unit holding m wavefronts, in units of one wavefront's time (2.8 us per
+// face, measured at 24^3 to 256^3 over segments of 1 to 48 faces): 1 up to three wavefronts
+// (the fourth shares a SIMD), 1.4 to 2.4 from four to eleven, 0.21 m from twelve on; a unit holds 12
+// wavefronts at a time (FP32 20), and more run in rounds of that size.  The plan takes the segment
+// length of least estimated time, at most the tuned one (cumc_tuning.seg).  Per y / z launch, 24-face
+// segments against the plan's: 48^3 46 -> 15.4 us, 96^3 86 -> 49, 128^3 132 / 108 -> 93 / 92,
+// torus 128x64x128 80 / 92 -> 50 / 53; 256^3 keeps 24.
+// ------------------------------------------------------------------------------------------
+struct WalkSet {
+    long waves;  // wavefronts per segment row
+    int faces;   // faces along the pencil
+};
+struct WalkPlan {
+    int sl;     // faces per segment
+    double us;  // estimated time of the launch
+};
+template <typename R>
+WalkSet walk_set(const Lay &L, int dir)
+{
+    const long pencils = (long)L.px * (dir == 2 ? flux_planes(L) : L.ny + 2);
+    return {(long)nblk(pencils, walk_block<R>()) * (walk_block<R>() / 64), (dir == 2 ? L.ny : L.nz) + 1};
+}
+static inline double cu_load(double m)
+{
+    if (m <= 0.0) return 0.0;
+    m = std::ceil(m);
+    return m <= 3.0 ? 1.0 : (m < 12.0 ? 1.4 + 0.14 * (m - 4.0) : 0.21 * m);
+}
+template <typename R>
+WalkPlan walk_plan(const WalkSet *w, int n, int max_sl)
+{
+    const double hold = sizeof(R) == 8 ? 12.0 : 20.0;
+    WalkPlan best{max_sl, 1e300};
+    int longest = 1;
+    for (int i = 0; i < n; i++) longest = w[i].faces > longest ? w[i].faces : longest;
+    for (int s = max_sl < longest ? max_sl : longest; s >= 1; s--) {
+        double waves = 0.0;
+        int sl = 1;
+        for (int i = 0; i < n; i++) {
+            const int ns = (w[i].faces + s - 1) / s, l = (w[i].faces + ns - 1) / ns;
+            waves += (double)w[i].waves * ns;
+            sl = l > sl ? l : sl;
+        }
+        const double per_cu = waves / 256.0, rounds = std::floor(per_cu / hold);
+        const double us = 3.0 + 2.8 * (sl + 1.3) * (rounds * 0.21 * hold + cu_load(per_cu - rounds * hold));
+        if (us < best.us) best = {s, us};
+    }
+    return best;
+}
+// the wave-parallel y sweep's time: 5.5 us and 3.3 us per 1000 wavefronts (measured 24^3 to 900^2)
+static inline double ylane_us(const Lay &L)
+{
+    return 5.5 + 0.0033 * 4.0 * ylane_groups(L) * ylane_segs(L) * flux_planes(L);
+}
+
 template <typename R, int RECON, int SOLVER>
 void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_dir)
 {
@@ -175,16 +235,18 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
     const int seg = ctx->seg;
     if (!only_dir || only_dir == 2) {
         mark(ctx, KC_FLUX_Y);
-        const int nseg = (L.ny + 1 + seg - 1) / seg;
-        if ((long)L.px * npl * nseg < YLANE_WALKERS && L.ny >= 16) {
-            // a 2D box whose pencil walks would leave most SIMDs idle: wave-parallel y sweep
+        const WalkSet w = walk_set<R>(L, 2);
+        const WalkPlan plan = walk_plan<R>(&w, 1, seg);
+        if (L.ny >= 16 && ylane_us(L) < plan.us) {
+            // few pencils: the wave-parallel y sweep
             const int gx = ylane_groups(L) * ylane_segs(L);
             hipLaunchKernelGGL((k_flux_ylane<R, RECON, SOLVER>), dim3(xcd_blocks(gx, npl)), dim3(256), 0, s, L, F, tb, M,
                                gx, npl);
         } else {
+            const int nseg = (L.ny + 1 + plan.sl - 1) / plan.sl;
             const int sl = (L.ny + 1 + nseg - 1) / nseg;
-            dim3 grid(nblk((long)L.px * npl, 128), nseg);
-            hipLaunchKernelGGL((k_flux_walk<R, 2, RECON, SOLVER>), grid, dim3(128), 0, s, L, F, tb, M, sl);
+            dim3 grid(nblk((long)L.px * npl, walk_block<R>()), nseg);
+            hipLaunchKernelGGL((k_flux_walk<R, 2, RECON, SOLVER>), grid, dim3(walk_block<R>()), 0, s, L, F, tb, M, sl);
         }
         mark(ctx, -1);
     }
@@ -192,10 +254,12 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
         mark(ctx, KC_FLUX_Z);
         // a z-collapsed view has one z face per column: faces 0 and 1 of the single cell are the
         // same face of its periodic images
-        const int nseg = L.zc1 ? 1 : (L.nz + 1 + seg - 1) / seg;
+        const WalkSet w = walk_set<R>(L, 3);
+        const int psl = L.zc1 ? 1 : walk_plan<R>(&w, 1, seg).sl;
+        const int nseg = L.zc1 ? 1 : (L.nz + 1 + psl - 1) / psl;
         const int sl = L.zc1 ? 1 : (L.nz + 1 + nseg - 1) / nseg;
-        dim3 grid(nblk((long)L.px * (L.ny + 2), 128), nseg);
-        hipLaunchKernelGGL((k_flux_walk<R, 3, RECON, SOLVER>), grid, dim3(128), 0, s, L, F, tb, M, sl);
+        dim3 grid(nblk((long)L.px * (L.ny + 2), walk_block<R>()), nseg);
+        hipLaunchKernelGGL((k_flux_walk<R, 3, RECON, SOLVER>), grid, dim3(walk_block<R>()), 0, s, L, F, tb, M, sl);
         mark(ctx, -1);
     }
 }

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void kb_flux_x(const BoxDesc *__restrict__ D, 
 }
 
 template <int DIR, int RECON>
-__global__ __launch_bounds__(128) void kb_flux_walk(const BoxDesc *__restrict__ D, const int *__restrict__ pre,
+__global__ __launch_bounds__(walk_block<double>()) void kb_flux_walk(const BoxDesc *__restrict__ D, const int *__restrict__ pre,
                                                     int nbox)
 {
     const int total = pre[nbox];
@@ -286,22 +286,22 @@ static void clear_graphs(cumc_batch *b)
     b->graphs.clear();
 }
 
-// tile counts of one box (in the addressing of its descriptor, d.L) under the current tuning
-static void box_tiles(const cumc_batch *b, BoxDesc &d, int cnt[P_N])
+// tile counts of one box (in the addressing of its descriptor, d.L) under the current tuning, with
+// y / z pencil segments of at most ysl / zsl faces
+static void box_tiles(const cumc_batch *b, BoxDesc &d, int ysl, int zsl, int cnt[P_N])
 {
     const Lay &L = d.L;
-    const int seg = b->tune.seg > 0 ? b->tune.seg : 24;
     const int zc = b->tune.zchunk > 0 ? b->tune.zchunk : 4;
     const long waves = ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES;
     d.fx_gx = (int)nblk(waves * 64, 256);
     cnt[P_FX] = d.fx_gx * flux_planes(L);
-    const int nsy = (L.ny + 1 + seg - 1) / seg;
+    const int nsy = (L.ny + 1 + ysl - 1) / ysl;
     d.fy_sl = (L.ny + 1 + nsy - 1) / nsy;
-    d.fy_gx = (int)nblk((long)L.px * flux_planes(L), 128);
+    d.fy_gx = (int)nblk((long)L.px * flux_planes(L), walk_block<double>());
     cnt[P_FY] = d.fy_gx * nsy;
-    const int nsz = L.zc1 ? 1 : (L.nz + 1 + seg - 1) / seg;  // one z face per column when collapsed
+    const int nsz = L.zc1 ? 1 : (L.nz + 1 + zsl - 1) / zsl;  // one z face per column when collapsed
     d.fz_sl = L.zc1 ? 1 : (L.nz + 1 + nsz - 1) / nsz;
-    d.fz_gx = (int)nblk((long)L.px * (L.ny + 2), 128);
+    d.fz_gx = (int)nblk((long)L.px * (L.ny + 2), walk_block<double>());
     cnt[P_FZ] = d.fz_gx * nsz;
     d.zc = zc;
     d.tw = b->tune.tile_w;
@@ -319,11 +319,22 @@ static int refresh(cumc_batch *b)
     const int nb = b->nbox;
     b->h_desc.assign(nb, BoxDesc{});
     b->h_pre.assign((size_t)P_N * (nb + 1), 0);
+    std::vector<View> views(nb);
+    std::vector<WalkSet> wy, wz;
+    for (int i = 0; i < nb; i++) {
+        cumc_ctx *c = b->box[i];
+        // an nz = 1 box steps in its z-collapsed view when it may (zcollapse_begin)
+        const View &v = views[i] = make_view(c, b->zfreeze ? c->zmode : zcollapse_begin(c));
+        wy.push_back(walk_set<double>(v.L, 2));
+        if (!v.L.zc1) wz.push_back(walk_set<double>(v.L, 3));
+    }
+    const int seg = b->tune.seg > 0 ? b->tune.seg : 24;
+    const int ysl = walk_plan<double>(wy.data(), nb, seg).sl;
+    const int zsl = wz.empty() ? seg : walk_plan<double>(wz.data(), (int)wz.size(), seg).sl;
     for (int i = 0; i < nb; i++) {
         cumc_ctx *c = b->box[i];
         BoxDesc &d = b->h_desc[i];
-        // an nz = 1 box steps in its z-collapsed view when it may (zcollapse_begin)
-        const View v = make_view(c, b->zfreeze ? c->zmode : zcollapse_begin(c));
+        const View &v = views[i];
         d.L = v.L;
         d.F = v.F;
         d.tb = tabs_of(c);
@@ -332,7 +343,7 @@ static int refresh(cumc_batch *b)
         d.Ub = v.Ub;
         d.sig = b->d_sig + i;
         int cnt[P_N];
-        box_tiles(b, d, cnt);
+        box_tiles(b, d, ysl, zsl, cnt);
         for (int p = 0; p < P_N; p++) b->h_pre[(size_t)p * (nb + 1) + i + 1] = b->h_pre[(size_t)p * (nb + 1) + i] + cnt[p];
     }
     for (int p = 0; p < P_N; p++) {
@@ -398,12 +409,12 @@ static void enqueue_fluxes_ecorn_b(cumc_batch *b)
     else hipLaunchKernelGGL((kb_flux_x<1>), dim3(grid_of(b, P_FX)), dim3(256), 0, s, D, pre_of(b, P_FX), nb);
     bmark(b, -1);
     bmark(b, P_FY);
-    if (ppm) hipLaunchKernelGGL((kb_flux_walk<2, 4>), dim3(grid_of(b, P_FY)), dim3(128), 0, s, D, pre_of(b, P_FY), nb);
-    else hipLaunchKernelGGL((kb_flux_walk<2, 1>), dim3(grid_of(b, P_FY)), dim3(128), 0, s, D, pre_of(b, P_FY), nb);
+    if (ppm) hipLaunchKernelGGL((kb_flux_walk<2, 4>), dim3(grid_of(b, P_FY)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FY), nb);
+    else hipLaunchKernelGGL((kb_flux_walk<2, 1>), dim3(grid_of(b, P_FY)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FY), nb);
     bmark(b, -1);
     bmark(b, P_FZ);
-    if (ppm) hipLaunchKernelGGL((kb_flux_walk<3, 4>), dim3(grid_of(b, P_FZ)), dim3(128), 0, s, D, pre_of(b, P_FZ), nb);
-    else hipLaunchKernelGGL((kb_flux_walk<3, 1>), dim3(grid_of(b, P_FZ)), dim3(128), 0, s, D, pre_of(b, P_FZ), nb);
+    if (ppm) hipLaunchKernelGGL((kb_flux_walk<3, 4>), dim3(grid_of(b, P_FZ)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FZ), nb);
+    else hipLaunchKernelGGL((kb_flux_walk<3, 1>), dim3(grid_of(b, P_FZ)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FZ), nb);
     bmark(b, -1);
     bmark(b, P_EC);
     hipLaunchKernelGGL(kb_ecorn, dim3(grid_of(b, P_EC)), dim3(256), 0, s, D, pre_of(b, P_EC), nb);

@@ -228,12 +228,10 @@ __global__ __launch_bounds__(256) void k_flux_x(Lay L, Fields<R> F, Tabs tb, Mod
 // of a workgroup take neighbouring pencils j, so the rows they load (stride px) meet in the same
 // 128-byte lines.  The same reconstruction and Riemann solve as the pencil walk, bit for bit.
 // Tile bx of plane l: 4-pencil group bx % njt (j in [0, nx+1]) of segment bx / njt.
-// A single context takes this form when its walks would run fewer than YLANE_WALKERS threads
-// (one wavefront per SIMD of the 256 CUs); with more walkers the walks keep up (the batched
-// 48-box workload, 1.2 M cells in 104 K walkers, measured 51.6 ms for 40 steps with this form in
-// XCD order against 51.7 ms with the walks, and 56.5 ms with this form in launch order).
+// A single context takes this form where walk_plan and ylane_us (ctx.hpp) expect it to be the
+// faster one: grids of a few thousand pencils' wavefronts (400^2: 17.5 us against 18.0 us; from 64^3
+// and 900^2 on the walks win, 24.4 against 27.8 and 46.7 against 59 us).
 // ------------------------------------------------------------------------------------------
-constexpr long YLANE_WALKERS = 1024L * 64;
 __host__ __device__ inline int ylane_groups(const Lay &L) { return (L.nx + 2 + 3) / 4; }
 __host__ __device__ inline int ylane_segs(const Lay &L) { return (L.ny + 1 + 2 + XS_FACES - 1) / XS_FACES; }
 
@@ -306,7 +304,13 @@ __device__ inline void flux_ylane_tile(const Lay &L, const Fields<R> &F, const T
 // each limiter call and each Riemann solve is computed exactly once.
 // (solver/spatial.f90:474-511 and :552-589)
 // ------------------------------------------------------------------------------------------
-// One 128-thread tile: bx covers px*(nt+2) pencils, segment by of seglen faces along DIR.
+// Threads of a walk workgroup.  FP64: one wavefront, so that the dispatcher spreads the wavefronts of
+// a small grid evenly (with two per workgroup a second workgroup on a compute unit shares the SIMDs of
+// the first: 48^3 in segments of 3 faces 20.5 us, with one 15.4 us; no difference on large grids).
+// FP32: two, whose neighbouring rows meet in one compute unit's cache (192^3 mixed 126 against 128 us).
+template <typename R>
+constexpr int walk_block() { return sizeof(R) == 8 ? 64 : 128; }
+// One walk_block-thread tile: bx covers px*(nt+2) pencils, segment by of seglen faces along DIR.
 template <typename R, int DIR, int RECON, int SOLVER = 2>
 __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Tabs &tb, const Model &M, int seglen,
                                       int bx, int by)
@@ -406,9 +410,14 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
             }
         }
     }
+    // the next cell's values and the face-normal B are loaded one cell ahead of their use: with one
+    // or two wavefronts per SIMD nothing else hides the latency
+    load7(s0 + 2, w3);
     for (int c = s0; c <= s1 + 1; c++) {
-        load7(c + 2, w3);
-        R vm[7], vp[7];
+        R wn[7], vm[7], vp[7];
+        load7(c + 3 < nd + 3 ? c + 3 : nd + 3, wn);
+        const unsigned gf = at(c - 1);
+        const R bn = ldi(sweep_p(F) + ibn * ps, gf);
         if constexpr (RECON == 5) {
 #pragma unroll
             for (int v = 0; v < 7; v++) weno5_edges<R>(wm[v], w0[v], w1[v], w2[v], w3[v], vm[v], vp[v]);
@@ -433,8 +442,6 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
         }
         if (c > s0) {
             // face c-1: left state = vp(c-1), right state = vm(c)
-            const unsigned gf = at(c - 1);
-            const R bn = ldi(sweep_p(F) + ibn * ps, gf);
             R fl[7];
             if (DIR == 2) {
                 // rotated frame n=y, t1=z, t2=x ; reconstructed cell B order (x, z)
@@ -471,12 +478,13 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
             vpp[v] = vp[v];
             w1[v] = w2[v];
             w2[v] = w3[v];
+            w3[v] = wn[v];
         }
     }
 }
 
 template <typename R, int DIR, int RECON, int SOLVER>
-__global__ __launch_bounds__(128) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
+__global__ __launch_bounds__(walk_block<R>()) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
 {
     flux_walk_tile<R, DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
 }
