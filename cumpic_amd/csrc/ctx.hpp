@@ -237,8 +237,10 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
         mark(ctx, KC_FLUX_Y);
         const WalkSet w = walk_set<R>(L, 2);
         const WalkPlan plan = walk_plan<R>(&w, 1, seg);
-        if (L.ny >= 16 && ylane_us(L) < plan.us) {
-            // few pencils: the wave-parallel y sweep
+        if (L.ny >= 16 && (sizeof(R) == 8 ? ylane_us(L) < plan.us : (long)L.px * npl * nblk(L.ny + 1, seg) < YLANE_WALKERS)) {
+            // few pencils: the wave-parallel y sweep.  FP32 keeps a fixed line, fewer walkers in segments
+            // of the tuned length than one wavefront per SIMD: its two forms contract different
+            // products, so the choice shows in the last FP32 bit
             const int gx = ylane_groups(L) * ylane_segs(L);
             hipLaunchKernelGGL((k_flux_ylane<R, RECON, SOLVER>), dim3(xcd_blocks(gx, npl)), dim3(256), 0, s, L, F, tb, M,
                                gx, npl);

@@ -116,9 +116,10 @@ constexpr int XS_FACES = 59;
 // (lane_up) or i + 1 (lane_down), the end lane keeping its own, as __shfl_up / __shfl_down with
 // delta 1 over 64 lanes.  FP64 values move by DPP whole-wave shifts (wave_shr:1 / wave_shl:1,
 // two VALU moves) instead of ds_bpermute through the LDS crossbar: the FP64 sweeps and the
-// reverse sweeps leave VALU cycles idle while they wait on the LDS.  FP32 values keep
-// ds_bpermute: the FP32 x sweep is VALU-bound and measured 10 % slower with the DPP moves.
-// Every lane of the wavefront must be active.
+// reverse sweeps leave VALU cycles idle while they wait on the LDS (shifts that fill the end lane
+// with zero need no copy of the old value, but made the 256^3 x sweep slower, 745 against 590 us).
+// FP32 values keep ds_bpermute: the FP32 x sweep is VALU-bound and measured 10 % slower with the DPP
+// moves.  Every lane of the wavefront must be active.
 __device__ inline int dpp_up1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xF, 0xF, false); }
 __device__ inline int dpp_dn1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xF, 0xF, false); }
 __device__ inline float lane_up(float v) { return __shfl_up(v, 1, 64); }
@@ -163,13 +164,15 @@ template <typename R, int RECON, int SOLVER = 2>
 __device__ inline void flux_x_tile(const Lay &L, const Fields<R> &F, const Tabs &tb, const Model &M, int bx, int l)
 {
     const int lane = threadIdx.x & 63;
-    const long wave = ((long)bx * blockDim.x + threadIdx.x) >> 6;
-    const long f = wave * XS_FACES + lane - 2;  // flattened (j+2) + k*px over rows k in [0, ny+1]
-    const long nload = (long)(L.ny + 4) * L.px;
+    // (a plane has fewer than 2^29 cells: 32-bit indices and a 32-bit division)
+    const int wave = (int)((bx * 256 + (int)threadIdx.x) >> 6);
+    const int f = wave * XS_FACES + lane - 2;  // flattened (j+2) + k*px over rows k in [0, ny+1]
+    const int px = (int)L.px, nload = (L.ny + 4) * px;
     const bool inr = (f >= 0) && (f < nload);
-    const long g = (long)(l + 2) * L.py + 2 * L.px + (inr ? f : 0);
-    const int k = inr ? (int)(f / L.px) : 0;
-    const int jj = inr ? (int)(f - (long)k * L.px) : 0;
+    const int fc = inr ? f : 0;
+    const long g = (long)(l + 2) * L.py + 2 * L.px + fc;
+    const int k = (int)((unsigned)fc / (unsigned)px);
+    const int jj = fc - k * px;
     const int j = jj - 2;
     const bool active = lane >= 2 && lane <= 60 && inr && k <= L.ny + 1 && j >= 0 && j <= L.nx;
     const int jc = j < -2 ? -2 : (j > L.nx + 3 ? L.nx + 3 : j);
@@ -232,6 +235,7 @@ __global__ __launch_bounds__(256) void k_flux_x(Lay L, Fields<R> F, Tabs tb, Mod
 // faster one: grids of a few thousand pencils' wavefronts (400^2: 17.5 us against 18.0 us; from 64^3
 // and 900^2 on the walks win, 24.4 against 27.8 and 46.7 against 59 us).
 // ------------------------------------------------------------------------------------------
+constexpr long YLANE_WALKERS = 1024L * 64;
 __host__ __device__ inline int ylane_groups(const Lay &L) { return (L.nx + 2 + 3) / 4; }
 __host__ __device__ inline int ylane_segs(const Lay &L) { return (L.ny + 1 + 2 + XS_FACES - 1) / XS_FACES; }
 
@@ -364,7 +368,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
                 const R bn = ldi(sweep_p(F) + ibn * ps, gf);
                 FaceState<R> sl{vp[0], vp[3], vp[1], vp[2], vp[4], bn, vp[5], vp[6]};
                 FaceState<R> sr{vm[0], vm[3], vm[1], vm[2], vm[4], bn, vm[5], vm[6]};
-                riemann_face<3, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
+                walk_face<3, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
                 R *o = F.F[2];
                 sti(o, gf, fl[0]);
                 sti(o + 1 * ps, gf, fl[2]);
@@ -447,7 +451,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
                 // rotated frame n=y, t1=z, t2=x ; reconstructed cell B order (x, z)
                 FaceState<R> sl{vpp[0], vpp[2], vpp[3], vpp[1], vpp[4], bn, vpp[6], vpp[5]};
                 FaceState<R> sr{vm[0], vm[2], vm[3], vm[1], vm[4], bn, vm[6], vm[5]};
-                riemann_face<2, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
+                walk_face<2, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
                 R *o = F.F[1];
                 sti(o, gf, fl[0]);
                 sti(o + 1 * ps, gf, fl[3]);
@@ -460,7 +464,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
                 // rotated frame n=z, t1=x, t2=y ; reconstructed cell B order (x, y)
                 FaceState<R> sl{vpp[0], vpp[3], vpp[1], vpp[2], vpp[4], bn, vpp[5], vpp[6]};
                 FaceState<R> sr{vm[0], vm[3], vm[1], vm[2], vm[4], bn, vm[5], vm[6]};
-                riemann_face<3, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
+                walk_face<3, R, SOLVER, RECON>(R(M.ggas), sl, sr, fl);
                 R *o = F.F[2];
                 sti(o, gf, fl[0]);
                 sti(o + 1 * ps, gf, fl[2]);
@@ -484,7 +488,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
 }
 
 template <typename R, int DIR, int RECON, int SOLVER>
-__global__ __launch_bounds__(walk_block<R>()) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
+__global__ __launch_bounds__(walk_block<R>(), sizeof(R) == 8 ? 3 : 1) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
 {
     flux_walk_tile<R, DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
 }

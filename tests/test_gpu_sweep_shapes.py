@@ -44,3 +44,48 @@ def test_step_matches_restatement(grid, recon):
     a, b = g.download(), o.get_state()
     for k in ("prim", "eps", "bcell"):
         assert_bitwise(a[k], b[k], k)
+
+
+# states whose quotients leave the range of the shared reciprocals in part of the box (fields below
+# 2^-300, densities and pressures below 2^-300 or above 2^300, zeros of both signs), so that a
+# wavefront takes both forms of the FP64 face
+EXTREMES = {
+    "tiny_b": lambda p, s: _scale(p, s, (5, 6, 7), 1e-95),
+    "subnormal_b": lambda p, s: _scale(p, s, (5, 6, 7), 1e-158),
+    "tiny_v": lambda p, s: _scale(p, s, (1, 2, 3), 1e-200),
+    "zero_v_and_b": lambda p, s: _scale(p, s, (1, 2, 3, 5, 6, 7), -0.0),
+    "tiny_rho_p": lambda p, s: _scale(p, s, (0, 4), 1e-95),
+    "huge_rho_p": lambda p, s: _scale(p, s, (0, 4), 1e95),
+    "zero_p": lambda p, s: _scale(p, s, (4,), 0.0),
+    "huge_b": lambda p, s: _scale(p, s, (5, 6, 7), 1e70),
+}
+
+
+def _scale(p, where, comps, factor):
+    for c in comps:
+        p.prim[where + (c,)] *= factor
+
+
+@pytest.mark.parametrize("recon", [4, 1])
+@pytest.mark.parametrize("kind", sorted(EXTREMES))
+def test_extreme_states_match_restatement(kind, recon):
+    from cumpic_amd.cumc import Solver
+    from oracle.oracle import Oracle
+    prob = _problem((21, 19, 17), recon)
+    EXTREMES[kind](prob, (slice(6, 14), slice(5, 15), slice(7, 17)))
+    prob.eps[...] = prob.prim[..., 4] / prob.prim[..., 0] / (prob.cfg.ggas - 1.0)
+    g, o = Solver.from_problem(prob), Oracle.from_problem(prob)
+    g.initial_update()
+    o.initial_update()
+    for d in (1, 2, 3):
+        a, b = g.sweep_flux(d), o.sweep_flux(d)
+        n = (prob.cfg.nx, prob.cfg.ny, prob.cfg.nz)
+        sl = tuple(slice(2, 3 + n[ax] + (ax + 1 != d)) for ax in (2, 1, 0))
+        assert_bitwise(a[sl], b[sl], f"{kind}: flux {d}")
+    dt = g.finddt()
+    assert dt == o.finddt()
+    g.rungekutta(dt)
+    o.rungekutta(dt)
+    a, b = g.download(), o.get_state()
+    for k in ("prim", "eps", "bcell"):
+        assert_bitwise(a[k], b[k], f"{kind}: {k}")
