@@ -157,7 +157,7 @@ void batch_after_run(cumc_batch *b, int nsteps);
 // ghost passes + torus clamp on the FP64 primitive planes (defined in cumc.hip) and on the
 // mixed form's FP32 planes (cumc_mixed.hip)
 void launch_ghost(cumc_ctx *ctx);
-void launch_ghost32(cumc_ctx *ctx);
+void launch_ghost32(cumc_ctx *ctx, double *dtnext);
 
 // ------------------------------------------------------------------------------------------
 // Segment length of the pencil walks.  A walk of sl faces takes about sl + 1.3 face times (warm-up
@@ -295,12 +295,26 @@ void launch_fluxes(cumc_ctx *ctx, const Fields<R> &F, int only_dir = 0)
     launch_fluxes<R>(ctx, ctx->L, F, only_dir);
 }
 
+// Planes a column thread of the stage tail (most: 2) and of the EMF kernel (most: 3) marches: at most
+// the tuned chunk.  A chunk saves the re-read of the plane below it (6 to 11 of the tail's 26 to 34
+// planes, out of cache) and costs a serial chain; and where even that leaves less than two workgroups
+// per compute unit (EMF: one), single planes shorten the chain.  Measured with chunks of 1 / 2 / 3 / 4:
+// tail 48^3 18.7 / 21.1 / 21.7 / 25.2 us, 128^3 222 / 220 / 222 / 224, torus 128x64x128 132 / 128 / 128 / 138,
+// 192^3 mixed 492 / 483 / 494 / 503; EMF 48^3 8.2 / 8.5 / 8.6 / 9.4, 128^3 84 / 74 / 71 / 71.
+static inline int column_chunk(const Lay &L, int tuned, int most, int tw, long fill)
+{
+    const int zc = tuned < most ? tuned : most;
+    return (long)col_tiles(L, tw) * zchunks(L, zc) < fill ? 1 : zc;
+}
+static inline int tail_chunk(const Lay &L, int tuned, int tw) { return column_chunk(L, tuned, 2, tw, 512); }
+static inline int ecorn_chunk(const Lay &L, int tuned, int tw) { return column_chunk(L, tuned, 3, tw, 256); }
+
 // comb: stage 1 writes, and stage 2 reads, the combined stage-2 input of a plain forward step
 // (rk_w2, comb_out in kernels.hpp); the mixed form combines only without sources and model hooks
 template <typename R, int STAGE, int COORD>
 void launch_tail_c(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, const double *Uin, double *Uout, bool comb)
 {
-    const int zc = ctx->zchunk, tw = ctx->tile_w;
+    const int tw = ctx->tile_w, zc = tail_chunk(L, ctx->zchunk, tw);
     const int gx = col_tiles(L, tw), gy = zchunks(L, zc);
     dim3 grid(xcd_blocks(gx, gy));
     Tabs tb = tabs_of(ctx);
@@ -348,8 +362,8 @@ static inline View make_view(const cumc_ctx *ctx, bool col)
     return v;
 }
 
-// ghost passes on the FP64 primitive planes of a view (defined in cumc.hip)
-void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F);
+// ghost fill of the FP64 primitive planes of a view (defined in cumc.hip)
+void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F, double *dtnext);
 // whether the next step runs in the z-collapsed view (enters it when allowed and the z ghost
 // planes check out), and the return of a collapsed state to the full layout (cumc.hip)
 bool zcollapse_begin(cumc_ctx *ctx);
@@ -364,7 +378,7 @@ void stage_l(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, double *Ub, int st
 {
     launch_fluxes<R>(ctx, L, F);
     mark(ctx, KC_ECORN);
-    const int zc = ctx->zchunk, tw = ctx->tile_w;
+    const int tw = ctx->tile_w, zc = ecorn_chunk(L, ctx->zchunk, tw);
     const int gx = col_tiles(L, tw), gy = zchunks(L, zc);
     hipLaunchKernelGGL((k_ecorn<R>), dim3(xcd_blocks(gx, gy)), dim3(256), 0, ctx->stream, L, F, gx, gy, zc, tw);
     mark(ctx, -1);
@@ -374,19 +388,15 @@ void stage_l(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, double *Ub, int st
     } else if (st == 2) {
         launch_tail<R, 2>(ctx, L, F, F.U1, Ub, comb);
     } else {
-        const double init = 1.0e10;
-        unsigned long long bits;
-        std::memcpy(&bits, &init, 8);
-        hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->stream, (unsigned long long *)(ctx->dt_dev + 1), bits, 1);
         launch_tail<R, 3>(ctx, L, F, Ub, F.U1, comb);
     }
     mark(ctx, -1);
     mark(ctx, KC_GHOST);
     if constexpr (sizeof(R) == 4) {
-        launch_ghost32(ctx);
+        launch_ghost32(ctx, st == 2 ? ctx->dt_dev + 1 : nullptr);
         ctx->p64_stale = true;
     } else {
-        launch_ghost_l(ctx, L, F);
+        launch_ghost_l(ctx, L, F, st == 2 ? ctx->dt_dev + 1 : nullptr);
     }
     mark(ctx, -1);
 }

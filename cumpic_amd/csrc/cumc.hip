@@ -429,25 +429,14 @@ extern "C" int cumc_download_noalloc(cumc_ctx *ctx, double *prim, double *eps, d
 // ---------------------------------------------------------------------------------------------
 // launch helpers
 // ---------------------------------------------------------------------------------------------
-void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F)
+void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F, double *dtnext)
 {
-    hipStream_t s = ctx->stream;
-    const long nx6 = L.nx + 6, ny6 = L.ny + 6;
-    hipLaunchKernelGGL(k_ghost<0>, dim3(nblk(ghost_threads<0>(L), 256)), dim3(256), 0, s, L, F, ctx->M);
-    hipLaunchKernelGGL(k_ghost<1>, dim3(nblk(ghost_threads<1>(L), 256)), dim3(256), 0, s, L, F, ctx->M);
-    // a z-collapsed view has no z pass: its z ghosts are the plane itself
-    if (!L.zc1) hipLaunchKernelGGL(k_ghost<2>, dim3(nblk(ghost_threads<2>(L), 256)), dim3(256), 0, s, L, F, ctx->M);
-    if (ctx->M.model == CUMC_MODEL_TORUS_CYN || ctx->M.model == CUMC_MODEL_TORUS_SPH) {
-        // inflow clamp on the R / r ghosts; torus_cyn also clamps the z ghosts
-        const long nyz = (long)(L.ny + 6) * (L.nz + 6) * 3, nxy = nx6 * ny6 * 3;
-        hipLaunchKernelGGL(k_custom_boundary_x<double>, dim3(nblk(nyz, 256)), dim3(256), 0, s, L, F.P);
-        if (ctx->M.model == CUMC_MODEL_TORUS_CYN)
-            hipLaunchKernelGGL(k_custom_boundary_z<double>, dim3(nblk(nxy, 256)), dim3(256), 0, s, L, F.P);
-    }
+    hipLaunchKernelGGL(k_ghost<double>, dim3(nblk(ghost_threads(L), 256)), dim3(256), 0, ctx->stream, L, F.P, F.EPS, F.BC,
+                       ctx->M, dtnext);
     if (!L.zc1) ctx->zfresh = true;
 }
 
-void launch_ghost(cumc_ctx *ctx) { launch_ghost_l(ctx, ctx->L, ctx->F64); }
+void launch_ghost(cumc_ctx *ctx) { launch_ghost_l(ctx, ctx->L, ctx->F64, nullptr); }
 
 // Enters the z-collapsed view when the context allows it and its state is a full-layout state
 // whose z ghost planes the last ghost fill wrote (zfresh) and whose two periodic B_z faces agree.

@@ -33,11 +33,11 @@ struct BoxDesc {
     int fx_gx;             // x sweep: tiles per plane
     int fy_gx, fy_sl;      // y sweep: tiles per segment row, faces per segment
     int fz_gx, fz_sl;      // z sweep
-    int c_gx, zc, tw;      // EMF / stage tail column tiles
+    int c_gx, zc, zt, tw;  // EMF / stage tail column tiles, planes per tile of either
     unsigned long long *sig;  // branch signature of the box (diagnostic build only)
 };
 
-enum { P_FX, P_FY, P_FZ, P_EC, P_TAIL, P_GX, P_GY, P_GZ, P_DT, P_N };
+enum { P_FX, P_FY, P_FZ, P_EC, P_TAIL, P_GHOST, P_DT, P_N };
 
 // largest b in [0, nbox) with pre[b] <= it  (pre[0] = 0 <= it < pre[nbox])
 __device__ inline int box_of(const int *pre, int nbox, int it)
@@ -142,20 +142,23 @@ __global__ __launch_bounds__(256) void kb_tail(const BoxDesc *__restrict__ D, co
         const double *Uin = STAGE == 1 ? F.U0 : (STAGE == 2 ? F.U1 : d.Ub);
         double *Uout = STAGE == 2 ? d.Ub : F.U1;
         tail_tile<double, STAGE, COORD, COMB>(d.L, F, d.tb, d.M, d.dt, Uin, Uout, (unsigned long long *)(d.dt + 1),
-                                        loc % d.c_gx, loc / d.c_gx, d.zc, d.tw);
+                                        loc % d.c_gx, loc / d.c_gx, d.zt, d.tw);
         BR_FLUSH(d, it);
     }
 }
 
-template <int AX>
-__global__ __launch_bounds__(256) void kb_ghost(const BoxDesc *__restrict__ D, const int *__restrict__ pre, int nbox)
+// reset (stage 2): the boxes' next-dt slots to the reduction identity 1e10 (rungekutta.f90:205), ahead of
+// stage 3's minimum
+__global__ __launch_bounds__(256) void kb_ghost(const BoxDesc *__restrict__ D, const int *__restrict__ pre, int nbox,
+                                                int reset)
 {
     const int total = pre[nbox];
     for (int it = blockIdx.x; it < total; it += gridDim.x) {
         const int b = box_of(pre, nbox, it);
         const long loc = it - pre[b];
         const BoxDesc &d = D[b];
-        ghost_thread<AX>(d.L, d.F, d.M, loc * blockDim.x + threadIdx.x);
+        if (reset && loc == 0 && threadIdx.x == 0) d.dt[1] = 1.0e10;
+        ghost_cell<double>(d.L, d.F.P, d.F.EPS, d.F.BC, d.M, loc * blockDim.x + threadIdx.x);
     }
 }
 
@@ -303,13 +306,13 @@ static void box_tiles(const cumc_batch *b, BoxDesc &d, int ysl, int zsl, int cnt
     d.fz_sl = L.zc1 ? 1 : (L.nz + 1 + nsz - 1) / nsz;
     d.fz_gx = (int)nblk((long)L.px * (L.ny + 2), walk_block<double>());
     cnt[P_FZ] = d.fz_gx * nsz;
-    d.zc = zc;
     d.tw = b->tune.tile_w;
+    d.zc = zc < 3 ? zc : 3;  // as ecorn_chunk and tail_chunk for a grid that fills the GPU
+    d.zt = zc < 2 ? zc : 2;
     d.c_gx = col_tiles(L, d.tw);
-    cnt[P_EC] = cnt[P_TAIL] = d.c_gx * zchunks(L, zc);
-    cnt[P_GX] = (int)nblk(ghost_threads<0>(L), 256);
-    cnt[P_GY] = (int)nblk(ghost_threads<1>(L), 256);
-    cnt[P_GZ] = (int)nblk(ghost_threads<2>(L), 256);
+    cnt[P_EC] = d.c_gx * zchunks(L, d.zc);
+    cnt[P_TAIL] = d.c_gx * zchunks(L, d.zt);
+    cnt[P_GHOST] = (int)nblk(ghost_threads(L), 256);
     cnt[P_DT] = (int)nblk((long)L.px * L.ny, 256);
 }
 
@@ -363,7 +366,7 @@ static inline const int *pre_of(const cumc_batch *b, int p) { return b->d_pre + 
 static inline unsigned grid_of(const cumc_batch *b, int p)
 {
     static const int tune_slot[P_N] = {CUMC_PH_FLUX_X, CUMC_PH_FLUX_Y, CUMC_PH_FLUX_Z, CUMC_PH_ECORN, CUMC_PH_TAIL,
-                                       CUMC_PH_GHOST,  CUMC_PH_GHOST,  CUMC_PH_GHOST,  CUMC_PH_FINDDT};
+                                       CUMC_PH_GHOST,  CUMC_PH_FINDDT};
     const int want = b->tune.blocks[tune_slot[p]];
     const int t = b->total[p];
     const int g = (want <= 0 || want > t) ? t : want;
@@ -428,7 +431,6 @@ static void enqueue_stage_b(cumc_batch *b, int st, int par, bool comb)
     const BoxDesc *D = b->d_desc;
     const int nb = b->nbox;
     enqueue_fluxes_ecorn_b(b);
-    if (st == 3) hipLaunchKernelGGL(kb_dt_reset, dim3(1), dim3(256), 0, s, D, nb);
     bmark(b, P_TAIL);
     if (comb && st < 3) {
         if (st == 1) launch_tail_b<1, true>(b, par);
@@ -439,11 +441,8 @@ static void enqueue_stage_b(cumc_batch *b, int st, int par, bool comb)
         else launch_tail_b<3, false>(b, par);
     }
     bmark(b, -1);
-    bmark(b, P_GX);
-    hipLaunchKernelGGL(kb_ghost<0>, dim3(grid_of(b, P_GX)), dim3(256), 0, s, D, pre_of(b, P_GX), nb);
-    hipLaunchKernelGGL(kb_ghost<1>, dim3(grid_of(b, P_GY)), dim3(256), 0, s, D, pre_of(b, P_GY), nb);
-    if (b->total[P_GZ] > 0)  // (no z pass when every box is z-collapsed)
-        hipLaunchKernelGGL(kb_ghost<2>, dim3(grid_of(b, P_GZ)), dim3(256), 0, s, D, pre_of(b, P_GZ), nb);
+    bmark(b, P_GHOST);
+    hipLaunchKernelGGL(kb_ghost, dim3(grid_of(b, P_GHOST)), dim3(256), 0, s, D, pre_of(b, P_GHOST), nb, st == 2 ? 1 : 0);
     bmark(b, -1);
 }
 
@@ -826,7 +825,7 @@ extern "C" int cumc_batch_autotune(cumc_batch *b, cumc_tuning *out)
         best.blocks[CUMC_PH_FLUX_Z] = pick[P_FZ];
         best.blocks[CUMC_PH_ECORN] = pick[P_EC];
         best.blocks[CUMC_PH_TAIL] = pick[P_TAIL];
-        best.blocks[CUMC_PH_GHOST] = pick[P_GX];
+        best.blocks[CUMC_PH_GHOST] = pick[P_GHOST];
         best.blocks[CUMC_PH_FINDDT] = pick[P_DT];
     }
     // restore every FP64 plane (so which of U0/U1 holds the state is as saved) and the dt slots

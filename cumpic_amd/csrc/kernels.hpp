@@ -1365,9 +1365,15 @@ static __global__ __launch_bounds__(256) void k_prim_from_u(Lay L, Fields<double
 }
 
 // ------------------------------------------------------------------------------------------
-// Ghost fill, one launch per pass in the reference's x -> y -> z order (boundary.f90:349-672 for
-// prim/bcell/transverse face B, boundary.f90:29-341 for eps), followed in each pass by UPDATE's
-// EOS on the ghost cells whose density and eps the pass finalises (update.f90:27-35).
+// Ghost fill in one launch.  The reference fills the ghosts in three passes, x -> y -> z
+// (boundary.f90:349-672 for prim/bcell/transverse face B, boundary.f90:29-341 for eps), each copying
+// from rows the passes before it filled, followed by UPDATE's EOS on the ghost cells
+// (update.f90:27-35) and by the torus inflow clamps (custom.f90:47-81).  A pass maps one index and
+// multiplies by +-1, so what the passes leave in a ghost cell is one interior value (or one face value
+// that no pass writes) times a product of signs: a thread per ghost cell takes it from there directly,
+// and no launch has to wait for another.  Three to five launches of 5 to 19 us became one: per stage
+// 800 cells 13.7 -> 7.5 us, 48^3 20.8 -> 9.4 us, 128^3 44 -> 28 us, 256^3 94 -> 84 us, cylindrical torus
+// 128x64x128 43 -> 18.5 us.
 // ------------------------------------------------------------------------------------------
 // source index along an axis of n interior cells for ghost g (1..3) on side s (0 low, 1 high);
 // periodic sources are wrapped so that n < NGHOST reproduces the sequential pass order
@@ -1390,141 +1396,102 @@ __device__ inline bool eps_y_outer(const int *bf, int *flag_eff)
     return false;
 }
 
-// number of ghost-fill threads of pass AX
-// (a z-collapsed view runs the x and y passes on its interior plane only and has no z pass: its
-// z ghosts are the plane itself)
-template <int AX>
+// ghost cells of a box: z slabs over the whole (j, k) plane, y slabs over the interior planes, x ghosts
+// of the interior rows (a z-collapsed view has its interior plane only: its z ghosts are the plane
+// itself)
 __host__ __device__ inline long ghost_threads(const Lay &L)
 {
-    const long nzb = L.zc1 ? 1 : L.nz + 1;
-    if (AX == 0) return (long)(L.ny + 1) * nzb * 6;
-    if (AX == 1) return (long)(L.nx + 6) * nzb * 6;
-    return L.zc1 ? 0 : (long)(L.nx + 6) * (L.ny + 6) * 6;
+    const long sx = L.nx + 6, sy = L.ny + 6, nzz = L.zc1 ? 1 : L.nz;
+    return 6 * ((L.zc1 ? 0 : sx * sy) + sx * nzz + (long)L.ny * nzz);
 }
 
-// One ghost cell of pass AX on the primitive planes P (8), EPS, BC (3) of element type T: the
-// FP64 state, or the FP32 copy of the mixed form (whose ghost pressure is formed in FP64 and
-// rounded, as the stage tail forms the interior one).
-template <int AX, typename T>
-__device__ inline void ghost_cells(const Lay &L, T *__restrict__ P, T *__restrict__ EPS, T *__restrict__ BC,
-                                   const Model &M, long t)
+// Ghost cell t of the primitive planes P (8), EPS, BC (3) of element type T: the FP64 state, or the
+// FP32 copy of the mixed form (whose ghost pressure is formed in FP64 and rounded, as the stage tail
+// forms the interior one).
+template <typename T>
+__device__ inline void ghost_cell(const Lay &L, T *P, T *EPS, T *BC, const Model &M, long t)
 {
-    // thread domain: (a, b) over the two other axes, g in 1..3, side in {0,1}
-    int na, nb, a0, b0;  // ranges [a0, a0+na) x [b0, b0+nb)
-    if (AX == 0) { a0 = 0; na = L.ny + 1; b0 = 0; nb = L.nz + 1; }           // k, l in [0,n]
-    else if (AX == 1) { a0 = -2; na = L.nx + 6; b0 = 0; nb = L.nz + 1; }     // j full, l in [0,n]
-    else { a0 = -2; na = L.nx + 6; b0 = -2; nb = L.ny + 6; }                 // j, k full
-    if (AX != 2 && L.zc1) { b0 = 1; nb = 1; }                                // the interior plane
-    const long per = (long)na * nb;
-    if (t >= per * 6) return;
-    int gs;  // 0..5 = (g-1)*2 + side
-    long r;
-    if (AX == 0) {
-        // x pass: the six ghost cells of one row are adjacent in memory, so let them be
-        // neighbouring threads
-        gs = (int)(t % 6);
-        r = t / 6;
+    const int sx = L.nx + 6, sy = L.ny + 6, nzz = L.zc1 ? 1 : L.nz;
+    const long tz = L.zc1 ? 0 : 6L * sx * sy, ty = 6L * sx * nzz, tx = 6L * L.ny * nzz;
+    if (t >= tz + ty + tx) return;
+    int j, k, l;
+    // ghost gs = (g-1)*2 + side along an axis of n cells
+    auto at = [](int gs, int n) { return (gs & 1) == 0 ? -(gs >> 1) : n + 1 + (gs >> 1); };
+    if (t < tz) {
+        const int per = sx * sy, r = (int)(t % per);
+        l = at((int)(t / per), L.nz);
+        j = r % sx - 2;
+        k = r / sx - 2;
+    } else if (t < tz + ty) {
+        const int u = (int)(t - tz), per = sx * nzz, r = u % per;
+        k = at(u / per, L.ny);
+        j = r % sx - 2;
+        l = r / sx + 1;
     } else {
-        gs = (int)(t / per);
-        r = t - (long)gs * per;
+        // the six ghost cells of one row are near each other in memory: neighbouring threads
+        const int u = (int)(t - tz - ty), r = u / 6;
+        j = at(u - r * 6, L.nx);
+        k = r % L.ny + 1;
+        l = r / L.ny + 1;
     }
-    const int g = gs / 2 + 1, side = gs & 1;
-    const int a = (int)(r % na) + a0, b = (int)(r / na) + b0;
-    const int n = AX == 0 ? L.nx : (AX == 1 ? L.ny : L.nz);
-    const int flag = M.bflag[2 * AX + side];
-    const int *fac = M.bfac[2 * AX + side];
-    const int dsti = side == 0 ? 1 - g : n + g;
-    const int srci = ghost_src(flag, side, g, n);
-    const long ps = L.ps;
-    long dst, src;
-    if (AX == 0) { dst = L.id(dsti, a, b); src = L.id(srci, a, b); }
-    else if (AX == 1) { dst = L.id(a, dsti, b); src = L.id(a, srci, b); }
-    else { dst = L.id(a, b, dsti); src = L.id(a, b, srci); }
-    const bool usef = flag >= 2;
-    // prim(1:5), bcell(1:3), transverse face B
+    // the cell each axis' pass copies from, and its parity factors where its flag takes them
+    const bool jg = j < 1 || j > L.nx, kg = k < 1 || k > L.ny, lg = !L.zc1 && (l < 1 || l > L.nz);
+    const int bx = j < 1 ? 0 : 1, by = k < 1 ? 2 : 3, bz = l < 1 ? 4 : 5;
+    const int gj = j < 1 ? 1 - j : j - L.nx, gk = k < 1 ? 1 - k : k - L.ny, gl = l < 1 ? 1 - l : l - L.nz;
+    const int sj = jg ? ghost_src(M.bflag[bx], bx & 1, gj, L.nx) : j;
+    const int sk = kg ? ghost_src(M.bflag[by], by & 1, gk, L.ny) : k;
+    const int sl = lg ? ghost_src(M.bflag[bz], bz & 1, gl, L.nz) : l;
+    const bool ux = jg && M.bflag[bx] >= 2, uy = kg && M.bflag[by] >= 2, uz = lg && M.bflag[bz] >= 2;
+    auto sgn = [&](T v, int i, bool x, bool y, bool z) {
+        if (!(x || y || z)) return v;
+        return (T)((x ? M.bfac[bx][i] : 1) * (y ? M.bfac[by][i] : 1) * (z ? M.bfac[bz][i] : 1)) * v;
+    };
+    const long ps = L.ps, dst = L.id(j, k, l), src = L.id(sj, sk, sl);
+    T v[5];
 #pragma unroll
-    for (int i = 0; i < 5; i++) P[dst + i * ps] = usef ? (T)fac[i] * P[src + i * ps] : P[src + i * ps];
+    for (int i = 0; i < 5; i++) v[i] = sgn(P[src + i * ps], i, ux, uy, uz);
 #pragma unroll
-    for (int c = 0; c < 3; c++)
-        BC[dst + c * ps] = usef ? (T)fac[5 + c] * BC[src + c * ps] : BC[src + c * ps];
-    const int tb1 = AX == 0 ? 6 : 5, tb2 = AX == 2 ? 6 : 7;
-    P[dst + tb1 * ps] = usef ? (T)fac[tb1] * P[src + tb1 * ps] : P[src + tb1 * ps];
-    P[dst + tb2 * ps] = usef ? (T)fac[tb2] * P[src + tb2 * ps] : P[src + tb2 * ps];
-    // eps (BOUNDARY1D ranges: x pass k,l in [1,n]; y pass l in [1,n]; z pass all)
-    bool final_region;
-    if (AX == 0) final_region = a >= 1 && a <= L.ny && b >= 1 && b <= L.nz;
-    else if (AX == 1) final_region = b >= 1 && b <= L.nz;
-    else final_region = true;
-    if (final_region) {
-        int ef = flag;
-        bool doit = true;
-        if (AX == 1 && side == 1) doit = eps_y_outer(M.bflag, &ef);
-        bool same_src = false;  // eps comes from the cell prim(1:5) came from
-        if (doit) {
-            const int es = ghost_src(ef, side, g, n);
-            same_src = es == srci;
-            long esrc;
-            if (AX == 0) esrc = L.id(es, a, b);
-            else if (AX == 1) esrc = L.id(a, es, b);
-            else esrc = L.id(a, b, es);
-            EPS[dst] = EPS[esrc];
+    for (int c = 0; c < 3; c++) BC[dst + c * ps] = sgn(BC[src + c * ps], 5 + c, ux, uy, uz);
+    // eps: the same cell, but for the y-outer side's own rule, which may also leave eps as it is
+    bool same = true;
+    long es = src;
+    if (kg && by == 3) {
+        int ef = 0;
+        if (eps_y_outer(M.bflag, &ef)) {
+            const int ek = ghost_src(ef, 1, gk, L.ny);
+            same = ek == sk;
+            es = L.id(sj, ek, sl);
+        } else {
+            same = false;
+            es = L.id(j, k, sl);
         }
-        // EOS.  With eps from the prim source cell the FP64 product equals the source pressure
-        // (formed by the same expression), which the FP32 planes then keep as copied.
-        if (sizeof(T) == 8 || !same_src) P[dst + 4 * ps] = (T)((double)P[dst] * (double)EPS[dst] * (M.ggas - 1.0));
     }
+    const T e = EPS[es];
+    if (es != dst) EPS[dst] = e;
+    // EOS.  With eps from the prim source cell the FP64 product equals the source pressure (formed by
+    // the same expression), which the FP32 planes keep as copied.
+    if (sizeof(T) == 8 || !same) v[4] = (T)((double)v[0] * (double)e * (M.ggas - 1.0));
+    // torus_cyn and torus_sph: no inflow through the R / r ghosts; torus_cyn: nor through the z ghosts
+    if (M.model != 0 && jg) v[1] = j < 1 ? fmin2<T>(v[1], T(0)) : fmax2<T>(v[1], T(0));
+    if (M.model == 1 && lg) v[3] = l < 1 ? fmin2<T>(v[3], T(0)) : fmax2<T>(v[3], T(0));
+#pragma unroll
+    for (int i = 0; i < 5; i++) P[dst + i * ps] = v[i];
+    // transverse face B: a pass takes the field along its own axis along only where that is transverse,
+    // on the rows [0, n] of the axes still to come
+    if (kg || lg) P[dst + 5 * ps] = sgn(P[L.id(j, sk, sl) + 5 * ps], 5, false, uy, uz);
+    const bool x6 = jg && k >= 0 && k <= L.ny;
+    if (x6 || lg) P[dst + 6 * ps] = sgn(P[L.id(x6 ? sj : j, k, sl) + 6 * ps], 6, ux && x6, false, uz);
+    if ((jg || kg) && l >= 0 && l <= L.nz) P[dst + 7 * ps] = sgn(P[L.id(sj, sk, l) + 7 * ps], 7, ux, uy, false);
 }
 
-template <int AX>
-__device__ inline void ghost_thread(const Lay &L, const Fields<double> &F, const Model &M, long t)
-{
-    ghost_cells<AX, double>(L, F.P, F.EPS, F.BC, M, t);
-}
-
-template <int AX>
-__global__ __launch_bounds__(256) void k_ghost(Lay L, Fields<double> F, Model M)
-{
-    ghost_thread<AX>(L, F, M, (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// ghost fill of the mixed form's FP32 primitive planes
-template <int AX>
-__global__ __launch_bounds__(256) void k_ghost32(Lay L, float *P32, float *EPS32, float *BC32, Model M)
-{
-    ghost_cells<AX, float>(L, P32, EPS32, BC32, M, (long)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// torus_cyn CUSTOM_BOUNDARY (custom.f90:47-81): no inflow through the R ghost zones ...
+// dtnext (null, or in stage 2): the next-dt slot, set to the reduction identity 1e10
+// (rungekutta.f90:205) ahead of stage 3, whose tail takes the minimum into it
 template <typename T>
-static __global__ __launch_bounds__(256) void k_custom_boundary_x(Lay L, T *P)
+__global__ __launch_bounds__(256) void k_ghost(Lay L, T *P, T *EPS, T *BC, Model M, double *dtnext)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long nyz = (long)(L.ny + 6) * (L.nz + 6);
-    if (t >= nyz * 3) return;
-    const int g = (int)(t / nyz) + 1;
-    const long r = t % nyz;
-    const int k = (int)(r % (L.ny + 6)) - 2, l = (int)(r / (L.ny + 6)) - 2;
-    T *vx = P + L.ps;
-    const long a = L.id(1 - g, k, l), b = L.id(L.nx + g, k, l);
-    vx[a] = fmin2<T>(vx[a], T(0));
-    vx[b] = fmax2<T>(vx[b], T(0));
-}
-
-// ... and through the z ghost zones
-template <typename T>
-static __global__ __launch_bounds__(256) void k_custom_boundary_z(Lay L, T *P)
-{
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ps = L.ps;
-    const long nxy = (long)(L.nx + 6) * (L.ny + 6);
-    if (t >= nxy * 3) return;
-    const int g = (int)(t / nxy) + 1;
-    const long r = t % nxy;
-    const int j = (int)(r % (L.nx + 6)) - 2, k = (int)(r / (L.nx + 6)) - 2;
-    T *vz = P + 3 * ps;
-    long a = L.id(j, k, 1 - g), b = L.id(j, k, L.nz + g);
-    vz[a] = fmin2<T>(vz[a], T(0));
-    vz[b] = fmax2<T>(vz[b], T(0));
+    if (t == 0 && dtnext) *dtnext = 1.0e10;
+    ghost_cell<T>(L, P, EPS, BC, M, t);
 }
 
 // ------------------------------------------------------------------------------------------
