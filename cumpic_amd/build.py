@@ -26,7 +26,7 @@ FP64_FLAGS = ["-ffp-contract=off", "-fno-fast-math"]
 MIXED_FLAGS = ["-ffp-contract=fast", "-fno-hip-fp32-correctly-rounded-divide-sqrt", "-fgpu-flush-denormals-to-zero"]
 
 UNITS = [("cumc.hip", FP64_FLAGS), ("cumc_mixed.hip", MIXED_FLAGS), ("cumc_batch.hip", FP64_FLAGS),
-         ("cumc_adjoint.hip", FP64_FLAGS)]
+         ("cumc_adjoint.hip", FP64_FLAGS), ("cumc_transfer.hip", FP64_FLAGS)]
 
 
 def _run(cmd):

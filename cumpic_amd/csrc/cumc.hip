@@ -12,7 +12,7 @@
 #include <string>
 #include <vector>
 
-#include "ctx.hpp"
+#include "transfer.hpp"
 
 // float instantiations live in cumc_mixed.hip (built with FP32 contraction and fast division)
 void stage_mixed(cumc_ctx *ctx, int st, bool comb);
@@ -93,6 +93,7 @@ extern "C" int cumc_create(const cumc_config *cfg, cumc_ctx **out)
         delete ctx;
         return CUMC_EHIP;
     }
+    staging_retain();
     Lay &L = ctx->L;
     L.nx = c.nx;
     L.ny = c.ny;
@@ -182,6 +183,7 @@ extern "C" int cumc_destroy(cumc_ctx *ctx)
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
+    staging_release();
     return CUMC_OK;
 }
 
@@ -290,36 +292,6 @@ extern "C" int cumc_set_grid(cumc_ctx *ctx, const double *xf, const double *yf, 
 }
 
 
-static int conv_in(cumc_ctx *ctx, const double *host, int nv, double *dst)
-{
-    const Lay &L = ctx->L;
-    const long ncell = (long)(L.nx + 6) * (L.ny + 6) * (L.nz + 6);
-    double *tmp = nullptr;
-    HIPCHK(ctx, hipMalloc(&tmp, (size_t)ncell * nv * sizeof(double)));
-    hipError_t e = hipMemcpyAsync(tmp, host, (size_t)ncell * nv * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_aos_to_soa, dim3(nblk(ncell, 256)), dim3(256), 0, ctx->stream, L, tmp, nv, dst);
-        e = hipStreamSynchronize(ctx->stream);
-    }
-    hipFree(tmp);
-    HIPCHK(ctx, e);
-    return CUMC_OK;
-}
-
-static int conv_out(cumc_ctx *ctx, const double *src, int nv, double *host)
-{
-    const Lay &L = ctx->L;
-    const long ncell = (long)(L.nx + 6) * (L.ny + 6) * (L.nz + 6);
-    double *tmp = nullptr;
-    HIPCHK(ctx, hipMalloc(&tmp, (size_t)ncell * nv * sizeof(double)));
-    hipLaunchKernelGGL(k_soa_to_aos, dim3(nblk(ncell, 256)), dim3(256), 0, ctx->stream, L, src, nv, tmp);
-    hipError_t e = hipMemcpyAsync(host, tmp, (size_t)ncell * nv * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(tmp);
-    HIPCHK(ctx, e);
-    return CUMC_OK;
-}
-
 extern "C" int cumc_upload(cumc_ctx *ctx, const double *prim, const double *eps)
 {
     if (!ctx || !prim || !eps) return CUMC_EINVAL;
@@ -330,9 +302,9 @@ extern "C" int cumc_upload(cumc_ctx *ctx, const double *prim, const double *eps)
     // bcell outside [1,n]^3 is read before the first BOUNDARY (as the reference's zero-initialised
     // array): a re-upload starts from the same zeros as a fresh context
     HIPCHK(ctx, hipMemsetAsync(ctx->F64.BC, 0, 3 * (size_t)ctx->L.ps * sizeof(double), ctx->stream));
-    int r = conv_in(ctx, prim, 8, ctx->F64.P);
+    const XferArray in[2] = {{ctx->F64.P, const_cast<double *>(prim), 8}, {ctx->F64.EPS, const_cast<double *>(eps), 1}};
+    const int r = transfer_in(ctx, in, 2);
     if (r) return r;
-    if ((r = conv_in(ctx, eps, 1, ctx->F64.EPS))) return r;
     ctx->p64_stale = false;
     prim_to_f32(ctx);
     HIPCHK(ctx, hipGetLastError());
@@ -343,13 +315,14 @@ extern "C" int cumc_upload(cumc_ctx *ctx, const double *prim, const double *eps)
 extern "C" int cumc_download(cumc_ctx *ctx, double *prim, double *eps, double *bcell)
 {
     if (!ctx) return CUMC_EINVAL;
-    int r;
     zexpand(ctx);
     sync_prim64(ctx);
-    if (prim && (r = conv_out(ctx, ctx->F64.P, 8, prim))) return r;
-    if (eps && (r = conv_out(ctx, ctx->F64.EPS, 1, eps))) return r;
-    if (bcell && (r = conv_out(ctx, ctx->F64.BC, 3, bcell))) return r;
-    return CUMC_OK;
+    XferArray out[3];
+    int n = 0;
+    if (prim) out[n++] = {ctx->F64.P, prim, 8};
+    if (eps) out[n++] = {ctx->F64.EPS, eps, 1};
+    if (bcell) out[n++] = {ctx->F64.BC, bcell, 3};
+    return transfer_out(ctx, out, n);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -23,7 +23,7 @@
 #include <vector>
 
 #include "adjoint.hpp"
-#include "ctx.hpp"
+#include "transfer.hpp"
 
 namespace {
 
@@ -1000,7 +1000,8 @@ __global__ __launch_bounds__(256) void kr_init_b(Lay L, AdjF A)
 struct cumc_tape {
     int nsteps = 0, every = 1;
     std::vector<double> dts;
-    double *mem = nullptr;     // one allocation
+    double *mem = nullptr;     // one allocation, of mem_words doubles
+    size_t mem_words = 0;
     double *init = nullptr;    // uploaded prim (8) + eps (1)
     double *ckpt = nullptr;    // nck states of SW planes: P 8, EPS 1, BC 3, U 8
     int nck = 0;
@@ -1142,6 +1143,15 @@ static void reverse_step(cumc_ctx *ctx, int i, double dt)
 // adjoint arrays and the three conserved-state adjoints
 static int tape_alloc(cumc_ctx *ctx, int nsteps, int every, bool zcollapse_ok = false, int sets = 1)
 {
+    // the last tape's allocation is kept where it serves (and is not four times too large): a training
+    // loop tapes the same map again and again, and 12 boxes of 64^2 to 192^2 took up to 0.3 s a pass to
+    // free and allocate their 20 GB
+    double *mem = nullptr;
+    size_t mem_words = 0;
+    if (ctx->tape) {
+        std::swap(mem, ctx->tape->mem);
+        mem_words = ctx->tape->mem_words;
+    }
     tape_release(ctx);
     // a single context's taped steps and their reversal run in the full layout (the stored states
     // keep their z ghost planes, which its reverse kernels read); the batched tape reverses
@@ -1158,10 +1168,18 @@ static int tape_alloc(cumc_ctx *ctx, int nsteps, int every, bool zcollapse_ok = 
     const size_t ps = ctx->L.ps;
     const size_t seg_states = sets > 1 ? (size_t)3 * (every + 1) * sets : (size_t)3 * every + 1;
     const size_t planes = 9 + (size_t)SW * tp->nck + (size_t)SW * seg_states + NADJ + 24;
-    if (hipMalloc(&tp->mem, planes * ps * sizeof(double)) != hipSuccess) {
-        tape_release(ctx);
-        return fail(ctx, CUMC_ENOMEM, "tape allocation");
+    const size_t words = planes * ps;
+    if (mem_words < words || mem_words / 4 > words) {
+        hipFree(mem);
+        mem = nullptr;
+        mem_words = words;
+        if (hipMalloc(&mem, words * sizeof(double)) != hipSuccess) {
+            tape_release(ctx);
+            return fail(ctx, CUMC_ENOMEM, "tape allocation");
+        }
     }
+    tp->mem = mem;
+    tp->mem_words = mem_words;
     double *p = tp->mem;
     auto take = [&](size_t n) { double *r = p; p += n * ps; return r; };
     tp->init = take(9);
@@ -1253,32 +1271,14 @@ extern "C" int cumc_tape_run(cumc_ctx *ctx, int nsteps, int every, const double 
 
 static int aos_into(cumc_ctx *ctx, const double *host, int nv, double *dst)
 {
-    const Lay &L = ctx->L;
-    const long ncell = (long)(L.nx + 6) * (L.ny + 6) * (L.nz + 6);
-    double *tmp = nullptr;
-    HIPCHK(ctx, hipMalloc(&tmp, (size_t)ncell * nv * sizeof(double)));
-    hipError_t e = hipMemcpyAsync(tmp, host, (size_t)ncell * nv * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_aos_to_soa, dim3(nblk(ncell, 256)), dim3(256), 0, ctx->stream, L, tmp, nv, dst);
-        e = hipStreamSynchronize(ctx->stream);
-    }
-    hipFree(tmp);
-    HIPCHK(ctx, e);
-    return CUMC_OK;
+    const XferArray a{dst, const_cast<double *>(host), nv};
+    return transfer_in(ctx, &a, 1);
 }
 
 static int soa_out(cumc_ctx *ctx, const double *src, int nv, double *host)
 {
-    const Lay &L = ctx->L;
-    const long ncell = (long)(L.nx + 6) * (L.ny + 6) * (L.nz + 6);
-    double *tmp = nullptr;
-    HIPCHK(ctx, hipMalloc(&tmp, (size_t)ncell * nv * sizeof(double)));
-    hipLaunchKernelGGL(k_soa_to_aos, dim3(nblk(ncell, 256)), dim3(256), 0, ctx->stream, L, src, nv, tmp);
-    hipError_t e = hipMemcpyAsync(host, tmp, (size_t)ncell * nv * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    hipFree(tmp);
-    HIPCHK(ctx, e);
-    return CUMC_OK;
+    const XferArray a{const_cast<double *>(src), host, nv};
+    return transfer_out(ctx, &a, 1);
 }
 
 extern "C" int cumc_tape_backward(cumc_ctx *ctx, const double *seed_prim, const double *seed_eps,
@@ -1627,6 +1627,7 @@ __global__ __launch_bounds__(256) void kbr_zfold_bc(Lay L, double *BC)
 }  // namespace
 
 struct batch_tape {
+    bool valid = false;  // a tape is recorded (the allocations and streams below outlive a failed tape_run)
     int nsteps = 0, every = 1, nck = 0, recon = 4;
     std::vector<AdjBox> h;
     AdjBox *d = nullptr;
@@ -1857,7 +1858,7 @@ extern "C" int cumc_batch_tape_run(cumc_batch *b, int nsteps, int every, const d
                 return CUMC_ENONFINITE;
             }
     for (int i = 0; i < nb; i++) BTCHK(b, hipStreamSynchronize(batch_box(b, i)->stream));
-    batch_tape_release(b);
+    if (batch_adj(b)) batch_adj(b)->valid = false;
     // two sets of segment buffers when the backward re-runs segments (it re-runs one segment
     // while it reverses the next)
     const int sets = nsteps > every ? 2 : 1;
@@ -1868,20 +1869,24 @@ extern "C" int cumc_batch_tape_run(cumc_batch *b, int nsteps, int every, const d
             return r;
         }
     }
-    batch_tape *bt = new batch_tape();
-    batch_adj(b) = bt;
+    // the descriptors, events and the second stream of the last tape serve again (their sizes follow
+    // the number of boxes)
+    if (!batch_adj(b)) batch_adj(b) = new batch_tape();
+    batch_tape *bt = batch_adj(b);
+    bt->valid = true;
+    bt->recompute_ms = 0.0;
     bt->nsteps = nsteps;
     bt->every = every;
     bt->nck = nsteps / every + 2;
     bt->recon = batch_box(b, 0)->cfg.recon;
     bt->h.assign(nb, AdjBox{});
-    BTCHK(b, hipMalloc(&bt->d, sizeof(AdjBox) * nb));
-    BTCHK(b, hipMalloc(&bt->pre, sizeof(int) * Q_N * (nb + 1)));
-    BTCHK(b, hipMalloc(&bt->d_full, sizeof(AdjBox) * nb));
-    BTCHK(b, hipMalloc(&bt->pre_full, sizeof(int) * Q_N * (nb + 1)));
-    BTCHK(b, hipEventCreate(&bt->e0));
-    BTCHK(b, hipEventCreate(&bt->e1));
-    BTCHK(b, hipStreamCreateWithFlags(&bt->s2, hipStreamNonBlocking));
+    if (!bt->d) BTCHK(b, hipMalloc(&bt->d, sizeof(AdjBox) * nb));
+    if (!bt->pre) BTCHK(b, hipMalloc(&bt->pre, sizeof(int) * Q_N * (nb + 1)));
+    if (!bt->d_full) BTCHK(b, hipMalloc(&bt->d_full, sizeof(AdjBox) * nb));
+    if (!bt->pre_full) BTCHK(b, hipMalloc(&bt->pre_full, sizeof(int) * Q_N * (nb + 1)));
+    if (!bt->e0) BTCHK(b, hipEventCreate(&bt->e0));
+    if (!bt->e1) BTCHK(b, hipEventCreate(&bt->e1));
+    if (!bt->s2) BTCHK(b, hipStreamCreateWithFlags(&bt->s2, hipStreamNonBlocking));
     int r = batch_refresh(b);
     if (r) return r;
     if ((r = bt_upload(b, bt))) return r;
@@ -1950,7 +1955,7 @@ extern "C" int cumc_batch_tape_backward(cumc_batch *b, const double *const *seed
 {
     if (!b) return CUMC_EINVAL;
     batch_tape *bt = batch_adj(b);
-    if (!bt) {
+    if (!bt || !bt->valid) {
         batch_err(b) = "cumc_batch_tape_run must precede cumc_batch_tape_backward";
         return CUMC_ESTATE;
     }
@@ -2090,7 +2095,7 @@ extern "C" int cumc_batch_tape_recompute_ms(cumc_batch *b, double *ms)
 {
     if (!b || !ms) return CUMC_EINVAL;
     batch_tape *bt = batch_adj(b);
-    if (!bt) return CUMC_ESTATE;
+    if (!bt || !bt->valid) return CUMC_ESTATE;
     *ms = bt->recompute_ms;
     return CUMC_OK;
 }

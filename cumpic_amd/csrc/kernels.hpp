@@ -1662,16 +1662,6 @@ static __global__ void k_zexpand(Lay L, Fields<double> F)
 // Layout conversion between the Fortran AoS arrays and the device planes
 // ------------------------------------------------------------------------------------------
 // aos[(cell)*nv + v] with cell = ((l+2)*(ny+6) + (k+2))*(nx+6) + (j+2)
-static __global__ void k_aos_to_soa(Lay L, const double *aos, int nv, double *soa)
-{
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long sx = L.nx + 6, sy = L.ny + 6, sz = L.nz + 6;
-    if (t >= sx * sy * sz) return;
-    const long jj = t % sx, kk = (t / sx) % sy, ll = t / (sx * sy);
-    const long g = ll * L.py + kk * L.px + jj;
-    for (int v = 0; v < nv; v++) soa[g + v * L.ps] = aos[t * nv + v];
-}
-
 static __global__ void k_soa_to_aos(Lay L, const double *soa, int nv, double *aos)
 {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
