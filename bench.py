@@ -81,7 +81,7 @@ KERNEL_IO_BYTES = {
     },
 }
 # kernels of the time step (per form) whose counter bytes make up the step traffic
-STEP_KERNELS = re.compile(r"k_(flux_x|flux_walk|ecorn|tail|stage_z|ghost32|ghost|fill_u64|custom_boundary)")
+STEP_KERNELS = re.compile(r"k_(flux_xyz|flux_x|flux_walk|ecorn|tail|stage_z|ghost32|ghost|fill_u64|custom_boundary)")
 
 
 def log(msg):
@@ -165,7 +165,10 @@ def pmc_traffic(ic_dir, form, steps=2, timeout=300):
 
 
 def kernel_class(name):
-    """Kernel class of a dispatch name (the classes of the library's HIP-event timing)."""
+    """Kernel class of a dispatch name (the classes of the library's HIP-event timing, and the three FP64
+    sweeps in one launch)."""
+    if "k_flux_xyz<" in name:
+        return "flux_xyz"
     if "k_flux_x<" in name:
         return "flux_x"
     if "k_flux_walk<" in name:

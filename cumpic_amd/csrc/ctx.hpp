@@ -167,7 +167,8 @@ void launch_ghost32(cumc_ctx *ctx, double *dtnext);
 // face, measured at 24^3 to 256^3 over segments of 1 to 48 faces): 1 up to three wavefronts
 // (the fourth shares a SIMD), 1.4 to 2.4 from four to eleven, 0.21 m from twelve on; a unit holds 12
 // wavefronts at a time (FP32 20), and more run in rounds of that size.  The plan takes the segment
-// length of least estimated time, at most the tuned one (cumc_tuning.seg).  Per y / z launch, 24-face
+// length of least estimated time, at most the tuned one (cumc_tuning.seg), for sweeps launched one by
+// one (the batch, the mixed form, profiling).  Per y / z launch, 24-face
 // segments against the plan's: 48^3 46 -> 15.4 us, 96^3 86 -> 49, 128^3 132 / 108 -> 93 / 92,
 // torus 128x64x128 80 / 92 -> 50 / 53; 256^3 keeps 24.
 // ------------------------------------------------------------------------------------------
@@ -177,7 +178,7 @@ struct WalkSet {
 };
 struct WalkPlan {
     int sl;     // faces per segment
-    double us;  // estimated time of the launch
+    double us;  // estimated time of a launch
 };
 template <typename R>
 WalkSet walk_set(const Lay &L, int dir)
@@ -212,10 +213,16 @@ WalkPlan walk_plan(const WalkSet *w, int n, int max_sl)
     }
     return best;
 }
-// the wave-parallel y sweep's time: 5.5 us and 3.3 us per 1000 wavefronts (measured 24^3 to 900^2)
-static inline double ylane_us(const Lay &L)
+// Faces per y / z segment where the three FP64 sweeps run in one launch (k_flux_xyz).  The launch
+// balances itself as long as one segment is short against the whole, about 2.5 us per 1024 wavefronts of
+// faces; so the segment grows with the faces.  Per step, segments of 1 / 3 / 6 / 12 / 24 faces:
+// 24^3 115 / 122 / 132 / 153 / 176 us, 64^3 322 / 277 / 265 / 292 / 315, 80^3 549 / 468 / 440 / 429 / 488,
+// 112^3 1335 / 1189 / 1144 / 1119 / 1111.
+static inline int one_launch_seg(const WalkSet w[3], int tuned)
 {
-    return 5.5 + 0.0033 * 4.0 * ylane_groups(L) * ylane_segs(L) * flux_planes(L);
+    const long face_waves = w[0].waves * w[0].faces + w[1].waves * w[1].faces + w[2].waves;
+    const long s = 1 + face_waves / 2400;
+    return (int)(s < tuned ? s : tuned);
 }
 
 template <typename R, int RECON, int SOLVER>
@@ -225,6 +232,26 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
     Tabs tb = tabs_of(ctx);
     const Model &M = ctx->M;
     const int npl = flux_planes(L);
+    if constexpr (sizeof(R) == 8) {
+        // (profiling times the three sweeps one by one)
+        if (!only_dir && !ctx->prof) {
+            const long xw = ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES;
+            const WalkSet w[3] = {walk_set<R>(L, 2), walk_set<R>(L, 3), {xw * npl, 1}};
+            SweepGrid G;
+            const int sl = one_launch_seg(w, ctx->seg);
+            const int ny = (w[0].faces + sl - 1) / sl, nz = L.zc1 ? 1 : (w[1].faces + sl - 1) / sl;
+            G.y_gx = (int)w[0].waves;
+            G.y_sl = (w[0].faces + ny - 1) / ny;
+            G.y_n = G.y_gx * ny;
+            G.z_gx = (int)w[1].waves;
+            G.z_sl = L.zc1 ? 1 : (w[1].faces + nz - 1) / nz;
+            G.z_n = G.z_gx * nz;
+            G.x_waves = (int)xw;
+            hipLaunchKernelGGL((k_flux_xyz<RECON, SOLVER>), dim3((unsigned)(G.y_n + G.z_n + xw * npl)), dim3(64), 0, s, L, F,
+                               tb, M, G);
+            return;
+        }
+    }
     if (!only_dir || only_dir == 1) {
         mark(ctx, KC_FLUX_X);
         const long waves = ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES;
@@ -237,13 +264,18 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
         mark(ctx, KC_FLUX_Y);
         const WalkSet w = walk_set<R>(L, 2);
         const WalkPlan plan = walk_plan<R>(&w, 1, seg);
-        if (L.ny >= 16 && (sizeof(R) == 8 ? ylane_us(L) < plan.us : (long)L.px * npl * nblk(L.ny + 1, seg) < YLANE_WALKERS)) {
-            // few pencils: the wave-parallel y sweep.  FP32 keeps a fixed line, fewer walkers in segments
-            // of the tuned length than one wavefront per SIMD: its two forms contract different
-            // products, so the choice shows in the last FP32 bit
-            const int gx = ylane_groups(L) * ylane_segs(L);
-            hipLaunchKernelGGL((k_flux_ylane<R, RECON, SOLVER>), dim3(xcd_blocks(gx, npl)), dim3(256), 0, s, L, F, tb, M,
-                               gx, npl);
+        bool lanes = false;
+        if constexpr (sizeof(R) == 4) {
+            // few pencils: the wave-parallel y sweep, below a fixed line in segments of the tuned length
+            // (the two FP32 forms contract different products, so the choice shows in the last bit)
+            lanes = L.ny >= 16 && (long)L.px * npl * nblk(L.ny + 1, seg) < YLANE_WALKERS;
+        }
+        if (lanes) {
+            if constexpr (sizeof(R) == 4) {
+                const int gx = ylane_groups(L) * ylane_segs(L);
+                hipLaunchKernelGGL((k_flux_ylane<R, RECON, SOLVER>), dim3(xcd_blocks(gx, npl)), dim3(256), 0, s, L, F, tb,
+                                   M, gx, npl);
+            }
         } else {
             const int nseg = (L.ny + 1 + plan.sl - 1) / plan.sl;
             const int sl = (L.ny + 1 + nseg - 1) / nseg;

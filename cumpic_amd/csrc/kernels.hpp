@@ -158,14 +158,12 @@ __device__ inline void recon_lane(const Tabs &tb, int ax, int jc, R c, R &vm, R 
     }
 }
 
-// One 256-thread tile of the x sweep: tile bx of plane l.  Tiles per plane:
-// ceil(ceil((ny+2)*px / XS_FACES) * 64 / 256), planes l in [0, nz+1].
+// One wavefront of the x sweep: number `wave` of the ceil((ny+2)*px / XS_FACES) of plane l in [0, nz+1].
 template <typename R, int RECON, int SOLVER = 2>
-__device__ inline void flux_x_tile(const Lay &L, const Fields<R> &F, const Tabs &tb, const Model &M, int bx, int l)
+__device__ inline void flux_x_wave(const Lay &L, const Fields<R> &F, const Tabs &tb, const Model &M, int wave, int l)
 {
     const int lane = threadIdx.x & 63;
     // (a plane has fewer than 2^29 cells: 32-bit indices and a 32-bit division)
-    const int wave = (int)((bx * 256 + (int)threadIdx.x) >> 6);
     const int f = wave * XS_FACES + lane - 2;  // flattened (j+2) + k*px over rows k in [0, ny+1]
     const int px = (int)L.px, nload = (L.ny + 4) * px;
     const bool inr = (f >= 0) && (f < nload);
@@ -218,6 +216,13 @@ __device__ inline void flux_x_tile(const Lay &L, const Fields<R> &F, const Tabs 
     }
 }
 
+// one 256-thread tile: four wavefronts
+template <typename R, int RECON, int SOLVER = 2>
+__device__ inline void flux_x_tile(const Lay &L, const Fields<R> &F, const Tabs &tb, const Model &M, int bx, int l)
+{
+    flux_x_wave<R, RECON, SOLVER>(L, F, tb, M, bx * 4 + (int)(threadIdx.x >> 6), l);
+}
+
 template <typename R, int RECON, int SOLVER>
 __global__ __launch_bounds__(256) void k_flux_x(Lay L, Fields<R> F, Tabs tb, Model M)
 {
@@ -231,9 +236,9 @@ __global__ __launch_bounds__(256) void k_flux_x(Lay L, Fields<R> F, Tabs tb, Mod
 // of a workgroup take neighbouring pencils j, so the rows they load (stride px) meet in the same
 // 128-byte lines.  The same reconstruction and Riemann solve as the pencil walk, bit for bit.
 // Tile bx of plane l: 4-pencil group bx % njt (j in [0, nx+1]) of segment bx / njt.
-// A single context takes this form where walk_plan and ylane_us (ctx.hpp) expect it to be the
-// faster one: grids of a few thousand pencils' wavefronts (400^2: 17.5 us against 18.0 us; from 64^3
-// and 900^2 on the walks win, 24.4 against 27.8 and 46.7 against 59 us).
+// The mixed form takes it where its walks in segments of the tuned length would run fewer than
+// YLANE_WALKERS threads (one wavefront per SIMD of the 256 CUs); the FP64 sweeps run in one launch
+// (k_flux_xyz), whose short walks are the faster ones.
 // ------------------------------------------------------------------------------------------
 constexpr long YLANE_WALKERS = 1024L * 64;
 __host__ __device__ inline int ylane_groups(const Lay &L) { return (L.nx + 2 + 3) / 4; }
@@ -491,6 +496,33 @@ template <typename R, int DIR, int RECON, int SOLVER>
 __global__ __launch_bounds__(walk_block<R>(), sizeof(R) == 8 ? 3 : 1) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
 {
     flux_walk_tile<R, DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
+}
+
+// The three FP64 sweeps in one launch: they read the same state and write their own planes, by itself
+// each is as long as its latency on a small grid (48^3: 13, 15 and 14 us), and the last wavefronts of
+// one leave the GPU idle until the next starts.  One wavefront per workgroup; the walks, the longer
+// ones, come first and the x wavefronts fill up (walks and x interleaved by slabs of planes, for the
+// cache's sake, cost 13 to 20 % up to 900^2 and 128x64x128 and gained 1 % at 256^3).  Per step, three
+// launches against one: 800 cells 117 -> 96 us, 400^2 210 -> 174, 64^3 335 -> 267, torus 128x64x128
+// 965 -> 872, 128^3 1679 -> 1605, 256^3 unchanged.
+// ------------------------------------------------------------------------------------------
+struct SweepGrid {
+    int y_gx, y_n, y_sl;  // y walks: tiles per segment row, tiles, faces per segment
+    int z_gx, z_n, z_sl;
+    int x_waves;          // x wavefronts per plane
+};
+template <int RECON, int SOLVER>
+__global__ __launch_bounds__(64, 3) void k_flux_xyz(Lay L, Fields<double> F, Tabs tb, Model M, SweepGrid G)
+{
+    int b = (int)blockIdx.x;
+    if (b < G.y_n) {
+        flux_walk_tile<double, 2, RECON, SOLVER>(L, F, tb, M, G.y_sl, b % G.y_gx, b / G.y_gx);
+    } else if ((b -= G.y_n) < G.z_n) {
+        flux_walk_tile<double, 3, RECON, SOLVER>(L, F, tb, M, G.z_sl, b % G.z_gx, b / G.z_gx);
+    } else {
+        b -= G.z_n;
+        flux_x_wave<double, RECON, SOLVER>(L, F, tb, M, b % G.x_waves, b / G.x_waves);
+    }
 }
 
 // ------------------------------------------------------------------------------------------

@@ -89,3 +89,19 @@ def test_extreme_states_match_restatement(kind, recon):
     a, b = g.download(), o.get_state()
     for k in ("prim", "eps", "bcell"):
         assert_bitwise(a[k], b[k], f"{kind}: {k}")
+
+
+@pytest.mark.parametrize("grid", [(7, 5, 1), (21, 18, 13), (130, 40, 33)])
+def test_one_launch_matches_separate_sweeps(grid):
+    """Sweeps timed one by one (profiling on) and in one launch give the same step."""
+    from cumpic_amd.cumc import Solver
+    states = []
+    for on in (False, True):
+        g = Solver.from_problem(_problem(grid, 4))
+        g.initial_update()
+        g.profile(on)
+        g.run(3)
+        states.append(g.download())
+        g.close()
+    for k in ("prim", "eps", "bcell"):
+        assert_bitwise(states[0][k], states[1][k], k)
