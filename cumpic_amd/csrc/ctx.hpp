@@ -168,17 +168,13 @@ void launch_ghost32(cumc_ctx *ctx, double *dtnext);
 // (the fourth shares a SIMD), 1.4 to 2.4 from four to eleven, 0.21 m from twelve on; a unit holds 12
 // wavefronts at a time (FP32 20), and more run in rounds of that size.  The plan takes the segment
 // length of least estimated time, at most the tuned one (cumc_tuning.seg), for sweeps launched one by
-// one (the batch, the mixed form, profiling).  Per y / z launch, 24-face
+// one (the mixed form, profiling).  Per y / z launch, 24-face
 // segments against the plan's: 48^3 46 -> 15.4 us, 96^3 86 -> 49, 128^3 132 / 108 -> 93 / 92,
 // torus 128x64x128 80 / 92 -> 50 / 53; 256^3 keeps 24.
 // ------------------------------------------------------------------------------------------
 struct WalkSet {
     long waves;  // wavefronts per segment row
     int faces;   // faces along the pencil
-};
-struct WalkPlan {
-    int sl;     // faces per segment
-    double us;  // estimated time of a launch
 };
 template <typename R>
 WalkSet walk_set(const Lay &L, int dir)
@@ -193,34 +189,35 @@ static inline double cu_load(double m)
     return m <= 3.0 ? 1.0 : (m < 12.0 ? 1.4 + 0.14 * (m - 4.0) : 0.21 * m);
 }
 template <typename R>
-WalkPlan walk_plan(const WalkSet *w, int n, int max_sl)
+int walk_plan(const WalkSet &w, int max_sl)
 {
     const double hold = sizeof(R) == 8 ? 12.0 : 20.0;
-    WalkPlan best{max_sl, 1e300};
-    int longest = 1;
-    for (int i = 0; i < n; i++) longest = w[i].faces > longest ? w[i].faces : longest;
-    for (int s = max_sl < longest ? max_sl : longest; s >= 1; s--) {
-        double waves = 0.0;
-        int sl = 1;
-        for (int i = 0; i < n; i++) {
-            const int ns = (w[i].faces + s - 1) / s, l = (w[i].faces + ns - 1) / ns;
-            waves += (double)w[i].waves * ns;
-            sl = l > sl ? l : sl;
-        }
-        const double per_cu = waves / 256.0, rounds = std::floor(per_cu / hold);
+    int best = max_sl;
+    double best_us = 1e300;
+    for (int s = max_sl < w.faces ? max_sl : w.faces; s >= 1; s--) {
+        const int ns = (w.faces + s - 1) / s, sl = (w.faces + ns - 1) / ns;
+        const double per_cu = (double)w.waves * ns / 256.0, rounds = std::floor(per_cu / hold);
         const double us = 3.0 + 2.8 * (sl + 1.3) * (rounds * 0.21 * hold + cu_load(per_cu - rounds * hold));
-        if (us < best.us) best = {s, us};
+        if (us < best_us) {
+            best = s;
+            best_us = us;
+        }
     }
     return best;
 }
-// Faces per y / z segment where the three FP64 sweeps run in one launch (k_flux_xyz).  The launch
+// Faces per y / z segment where the three FP64 sweeps run in one launch (k_flux_xyz, kb_flux_xyz).  The launch
 // balances itself as long as one segment is short against the whole, about 2.5 us per 1024 wavefronts of
 // faces; so the segment grows with the faces.  Per step, segments of 1 / 3 / 6 / 12 / 24 faces:
 // 24^3 115 / 122 / 132 / 153 / 176 us, 64^3 322 / 277 / 265 / 292 / 315, 80^3 549 / 468 / 440 / 429 / 488,
 // 112^3 1335 / 1189 / 1144 / 1119 / 1111.
-static inline int one_launch_seg(const WalkSet w[3], int tuned)
+static inline long x_waves(const Lay &L) { return ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES; }
+static inline long sweep_face_waves(const Lay &L)
 {
-    const long face_waves = w[0].waves * w[0].faces + w[1].waves * w[1].faces + w[2].waves;
+    const WalkSet y = walk_set<double>(L, 2), z = walk_set<double>(L, 3);
+    return y.waves * y.faces + z.waves * z.faces + x_waves(L) * flux_planes(L);
+}
+static inline int one_launch_seg(long face_waves, int tuned)
+{
     const long s = 1 + face_waves / 2400;
     return (int)(s < tuned ? s : tuned);
 }
@@ -235,16 +232,16 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
     if constexpr (sizeof(R) == 8) {
         // (profiling times the three sweeps one by one)
         if (!only_dir && !ctx->prof) {
-            const long xw = ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES;
-            const WalkSet w[3] = {walk_set<R>(L, 2), walk_set<R>(L, 3), {xw * npl, 1}};
+            const long xw = x_waves(L);
+            const WalkSet wy = walk_set<R>(L, 2), wz = walk_set<R>(L, 3);
             SweepGrid G;
-            const int sl = one_launch_seg(w, ctx->seg);
-            const int ny = (w[0].faces + sl - 1) / sl, nz = L.zc1 ? 1 : (w[1].faces + sl - 1) / sl;
-            G.y_gx = (int)w[0].waves;
-            G.y_sl = (w[0].faces + ny - 1) / ny;
+            const int sl = one_launch_seg(sweep_face_waves(L), ctx->seg);
+            const int ny = (wy.faces + sl - 1) / sl, nz = L.zc1 ? 1 : (wz.faces + sl - 1) / sl;
+            G.y_gx = (int)wy.waves;
+            G.y_sl = (wy.faces + ny - 1) / ny;
             G.y_n = G.y_gx * ny;
-            G.z_gx = (int)w[1].waves;
-            G.z_sl = L.zc1 ? 1 : (w[1].faces + nz - 1) / nz;
+            G.z_gx = (int)wz.waves;
+            G.z_sl = L.zc1 ? 1 : (wz.faces + nz - 1) / nz;
             G.z_n = G.z_gx * nz;
             G.x_waves = (int)xw;
             hipLaunchKernelGGL((k_flux_xyz<RECON, SOLVER>), dim3((unsigned)(G.y_n + G.z_n + xw * npl)), dim3(64), 0, s, L, F,
@@ -254,16 +251,14 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
     }
     if (!only_dir || only_dir == 1) {
         mark(ctx, KC_FLUX_X);
-        const long waves = ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES;
-        dim3 grid(nblk(waves * 64, 256), npl);
+        dim3 grid(nblk(x_waves(L) * 64, 256), npl);
         hipLaunchKernelGGL((k_flux_x<R, RECON, SOLVER>), grid, dim3(256), 0, s, L, F, tb, M);
         mark(ctx, -1);
     }
     const int seg = ctx->seg;
     if (!only_dir || only_dir == 2) {
         mark(ctx, KC_FLUX_Y);
-        const WalkSet w = walk_set<R>(L, 2);
-        const WalkPlan plan = walk_plan<R>(&w, 1, seg);
+        const int psl = walk_plan<R>(walk_set<R>(L, 2), seg);
         bool lanes = false;
         if constexpr (sizeof(R) == 4) {
             // few pencils: the wave-parallel y sweep, below a fixed line in segments of the tuned length
@@ -277,7 +272,7 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
                                    M, gx, npl);
             }
         } else {
-            const int nseg = (L.ny + 1 + plan.sl - 1) / plan.sl;
+            const int nseg = (L.ny + 1 + psl - 1) / psl;
             const int sl = (L.ny + 1 + nseg - 1) / nseg;
             dim3 grid(nblk((long)L.px * npl, walk_block<R>()), nseg);
             hipLaunchKernelGGL((k_flux_walk<R, 2, RECON, SOLVER>), grid, dim3(walk_block<R>()), 0, s, L, F, tb, M, sl);
@@ -288,8 +283,7 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
         mark(ctx, KC_FLUX_Z);
         // a z-collapsed view has one z face per column: faces 0 and 1 of the single cell are the
         // same face of its periodic images
-        const WalkSet w = walk_set<R>(L, 3);
-        const int psl = L.zc1 ? 1 : walk_plan<R>(&w, 1, seg).sl;
+        const int psl = L.zc1 ? 1 : walk_plan<R>(walk_set<R>(L, 3), seg);
         const int nseg = L.zc1 ? 1 : (L.nz + 1 + psl - 1) / psl;
         const int sl = L.zc1 ? 1 : (L.nz + 1 + nseg - 1) / nseg;
         dim3 grid(nblk((long)L.px * (L.ny + 2), walk_block<R>()), nseg);

@@ -30,7 +30,7 @@ struct BoxDesc {
     Model M;
     double *dt;  // [0] current step, [1] next step (stage-3 reduction target)
     double *Ub;
-    int fx_gx;             // x sweep: tiles per plane
+    int fx_gx;             // x sweep: wavefronts per plane
     int fy_gx, fy_sl;      // y sweep: tiles per segment row, faces per segment
     int fz_gx, fz_sl;      // z sweep
     int c_gx, zc, zt, tw;  // EMF / stage tail column tiles, planes per tile of either
@@ -85,33 +85,28 @@ __device__ inline void br_flush(unsigned long long *sig, int it)
 #define BR_FLUSH(d, it) ((void)0)
 #endif
 
+// The three sweeps of every box in one launch, as k_flux_xyz for one grid: the y tiles of all boxes,
+// then their z tiles, then the x wavefronts, one wavefront per workgroup (a launch each drains
+// before the next starts, and the y walks, the few of a flat box, last longest).  48 flat boxes of 64 to
+// 256 cells a side 161 -> 128 us per stage (step 970 -> 856 us), 12 of 64 to 192 52 -> 41 us (278 -> 240).
 template <int RECON>
-__global__ __launch_bounds__(256) void kb_flux_x(const BoxDesc *__restrict__ D, const int *__restrict__ pre, int nbox)
+__global__ __launch_bounds__(64, 3) void kb_flux_xyz(const BoxDesc *__restrict__ D, const int *__restrict__ prex,
+                                                    const int *__restrict__ prey, const int *__restrict__ prez, int nbox)
 {
-    const int total = pre[nbox];
+    const int ny = prey[nbox], nyz = ny + prez[nbox], total = nyz + prex[nbox];
     BR_START();
     for (int it = blockIdx.x; it < total; it += gridDim.x) {
-        const int b = box_of(pre, nbox, it);
-        const int loc = it - pre[b];
+        const int *pre = it < ny ? prey : (it < nyz ? prez : prex);
+        const int t = it - (it < ny ? 0 : (it < nyz ? ny : nyz));
+        const int b = box_of(pre, nbox, t);
+        const int loc = t - pre[b];
         const BoxDesc &d = D[b];
-        flux_x_tile<double, RECON>(d.L, d.F, d.tb, d.M, loc % d.fx_gx, loc / d.fx_gx);
-        BR_FLUSH(d, it);
-    }
-}
-
-template <int DIR, int RECON>
-__global__ __launch_bounds__(walk_block<double>()) void kb_flux_walk(const BoxDesc *__restrict__ D, const int *__restrict__ pre,
-                                                    int nbox)
-{
-    const int total = pre[nbox];
-    BR_START();
-    for (int it = blockIdx.x; it < total; it += gridDim.x) {
-        const int b = box_of(pre, nbox, it);
-        const int loc = it - pre[b];
-        const BoxDesc &d = D[b];
-        const int gx = DIR == 2 ? d.fy_gx : d.fz_gx;
-        const int sl = DIR == 2 ? d.fy_sl : d.fz_sl;
-        flux_walk_tile<double, DIR, RECON>(d.L, d.F, d.tb, d.M, sl, loc % gx, loc / gx);
+        if (it < ny)
+            flux_walk_tile<double, 2, RECON>(d.L, d.F, d.tb, d.M, d.fy_sl, loc % d.fy_gx, loc / d.fy_gx);
+        else if (it < nyz)
+            flux_walk_tile<double, 3, RECON>(d.L, d.F, d.tb, d.M, d.fz_sl, loc % d.fz_gx, loc / d.fz_gx);
+        else
+            flux_x_wave<double, RECON>(d.L, d.F, d.tb, d.M, loc % d.fx_gx, loc / d.fx_gx);
         BR_FLUSH(d, it);
     }
 }
@@ -290,19 +285,18 @@ static void clear_graphs(cumc_batch *b)
 }
 
 // tile counts of one box (in the addressing of its descriptor, d.L) under the current tuning, with
-// y / z pencil segments of at most ysl / zsl faces
-static void box_tiles(const cumc_batch *b, BoxDesc &d, int ysl, int zsl, int cnt[P_N])
+// y / z pencil segments of at most sl faces
+static void box_tiles(const cumc_batch *b, BoxDesc &d, int sl, int cnt[P_N])
 {
     const Lay &L = d.L;
     const int zc = b->tune.zchunk > 0 ? b->tune.zchunk : 4;
-    const long waves = ((long)(L.ny + 2) * L.px + XS_FACES - 1) / XS_FACES;
-    d.fx_gx = (int)nblk(waves * 64, 256);
+    d.fx_gx = (int)x_waves(L);
     cnt[P_FX] = d.fx_gx * flux_planes(L);
-    const int nsy = (L.ny + 1 + ysl - 1) / ysl;
+    const int nsy = (L.ny + 1 + sl - 1) / sl;
     d.fy_sl = (L.ny + 1 + nsy - 1) / nsy;
     d.fy_gx = (int)nblk((long)L.px * flux_planes(L), walk_block<double>());
     cnt[P_FY] = d.fy_gx * nsy;
-    const int nsz = L.zc1 ? 1 : (L.nz + 1 + zsl - 1) / zsl;  // one z face per column when collapsed
+    const int nsz = L.zc1 ? 1 : (L.nz + 1 + sl - 1) / sl;  // one z face per column when collapsed
     d.fz_sl = L.zc1 ? 1 : (L.nz + 1 + nsz - 1) / nsz;
     d.fz_gx = (int)nblk((long)L.px * (L.ny + 2), walk_block<double>());
     cnt[P_FZ] = d.fz_gx * nsz;
@@ -323,17 +317,15 @@ static int refresh(cumc_batch *b)
     b->h_desc.assign(nb, BoxDesc{});
     b->h_pre.assign((size_t)P_N * (nb + 1), 0);
     std::vector<View> views(nb);
-    std::vector<WalkSet> wy, wz;
+    long face_waves = 0;
     for (int i = 0; i < nb; i++) {
         cumc_ctx *c = b->box[i];
         // an nz = 1 box steps in its z-collapsed view when it may (zcollapse_begin)
         const View &v = views[i] = make_view(c, b->zfreeze ? c->zmode : zcollapse_begin(c));
-        wy.push_back(walk_set<double>(v.L, 2));
-        if (!v.L.zc1) wz.push_back(walk_set<double>(v.L, 3));
+        face_waves += sweep_face_waves(v.L);
     }
     const int seg = b->tune.seg > 0 ? b->tune.seg : 24;
-    const int ysl = walk_plan<double>(wy.data(), nb, seg).sl;
-    const int zsl = wz.empty() ? seg : walk_plan<double>(wz.data(), (int)wz.size(), seg).sl;
+    const int sl = one_launch_seg(face_waves, seg);
     for (int i = 0; i < nb; i++) {
         cumc_ctx *c = b->box[i];
         BoxDesc &d = b->h_desc[i];
@@ -346,7 +338,7 @@ static int refresh(cumc_batch *b)
         d.Ub = v.Ub;
         d.sig = b->d_sig + i;
         int cnt[P_N];
-        box_tiles(b, d, ysl, zsl, cnt);
+        box_tiles(b, d, sl, cnt);
         for (int p = 0; p < P_N; p++) b->h_pre[(size_t)p * (nb + 1) + i + 1] = b->h_pre[(size_t)p * (nb + 1) + i] + cnt[p];
     }
     for (int p = 0; p < P_N; p++) {
@@ -354,6 +346,8 @@ static int refresh(cumc_batch *b)
         if (t > 0x7fffffffL) return bfail(b, CUMC_EINVAL, "batch work list exceeds 2^31 tiles");
         b->total[p] = (int)t;
     }
+    if ((long)b->total[P_FX] + b->total[P_FY] + b->total[P_FZ] > 0x7fffffffL)
+        return bfail(b, CUMC_EINVAL, "batch work list exceeds 2^31 tiles");
     BCHK(b, hipMemcpyAsync(b->d_desc, b->h_desc.data(), sizeof(BoxDesc) * nb, hipMemcpyHostToDevice, b->stream));
     BCHK(b, hipMemcpyAsync(b->d_pre, b->h_pre.data(), sizeof(int) * b->h_pre.size(), hipMemcpyHostToDevice, b->stream));
     BCHK(b, hipStreamSynchronize(b->stream));
@@ -408,16 +402,10 @@ static void enqueue_fluxes_ecorn_b(cumc_batch *b)
     const int nb = b->nbox;
     const bool ppm = b->recon == CUMC_PPMC;
     bmark(b, P_FX);
-    if (ppm) hipLaunchKernelGGL((kb_flux_x<4>), dim3(grid_of(b, P_FX)), dim3(256), 0, s, D, pre_of(b, P_FX), nb);
-    else hipLaunchKernelGGL((kb_flux_x<1>), dim3(grid_of(b, P_FX)), dim3(256), 0, s, D, pre_of(b, P_FX), nb);
-    bmark(b, -1);
-    bmark(b, P_FY);
-    if (ppm) hipLaunchKernelGGL((kb_flux_walk<2, 4>), dim3(grid_of(b, P_FY)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FY), nb);
-    else hipLaunchKernelGGL((kb_flux_walk<2, 1>), dim3(grid_of(b, P_FY)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FY), nb);
-    bmark(b, -1);
-    bmark(b, P_FZ);
-    if (ppm) hipLaunchKernelGGL((kb_flux_walk<3, 4>), dim3(grid_of(b, P_FZ)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FZ), nb);
-    else hipLaunchKernelGGL((kb_flux_walk<3, 1>), dim3(grid_of(b, P_FZ)), dim3(walk_block<double>()), 0, s, D, pre_of(b, P_FZ), nb);
+    const unsigned g = grid_of(b, P_FX) + grid_of(b, P_FY) + grid_of(b, P_FZ);
+    const int *px = pre_of(b, P_FX), *py = pre_of(b, P_FY), *pz = pre_of(b, P_FZ);
+    if (ppm) hipLaunchKernelGGL((kb_flux_xyz<4>), dim3(g), dim3(64), 0, s, D, px, py, pz, nb);
+    else hipLaunchKernelGGL((kb_flux_xyz<1>), dim3(g), dim3(64), 0, s, D, px, py, pz, nb);
     bmark(b, -1);
     bmark(b, P_EC);
     hipLaunchKernelGGL(kb_ecorn, dim3(grid_of(b, P_EC)), dim3(256), 0, s, D, pre_of(b, P_EC), nb);
@@ -763,7 +751,7 @@ extern "C" int cumc_batch_autotune(cumc_batch *b, cumc_tuning *out)
             for (int p = 0; p < CUMC_PH_N; p++) t.blocks[p] = 0;
             double ph[P_N];
             if ((rc = time_candidate(b, t, ph))) break;
-            const double v = ph[P_FY] + ph[P_FZ];
+            const double v = ph[P_FX];
             if (v < bestt) {
                 bestt = v;
                 best.seg = sg;
@@ -803,7 +791,7 @@ extern "C" int cumc_batch_autotune(cumc_batch *b, cumc_tuning *out)
             }
         }
     }
-    // 3) persistent workgroups per phase
+    // 3) persistent workgroups per phase (the sweeps are one launch, timed as the x sweep's phase)
     if (rc == CUMC_OK) {
         const int cands[] = {0, 256, 512, 1024, 2048, 4096};
         double bt[P_N];
@@ -821,8 +809,8 @@ extern "C" int cumc_batch_autotune(cumc_batch *b, cumc_tuning *out)
                 }
         }
         best.blocks[CUMC_PH_FLUX_X] = pick[P_FX];
-        best.blocks[CUMC_PH_FLUX_Y] = pick[P_FY];
-        best.blocks[CUMC_PH_FLUX_Z] = pick[P_FZ];
+        best.blocks[CUMC_PH_FLUX_Y] = pick[P_FX];
+        best.blocks[CUMC_PH_FLUX_Z] = pick[P_FX];
         best.blocks[CUMC_PH_ECORN] = pick[P_EC];
         best.blocks[CUMC_PH_TAIL] = pick[P_TAIL];
         best.blocks[CUMC_PH_GHOST] = pick[P_GHOST];
