@@ -28,6 +28,9 @@ struct cumc_ctx {
     double *tab[3] = {nullptr, nullptr, nullptr};
     float *tabf[3] = {nullptr, nullptr, nullptr};
     double *dt_dev = nullptr;           // [0] dt of the current step, [1] dt found by stage 3
+    // pinned word through which a run's steps hand the next dt to the host (finddt_published);
+    // dt_pub is its device address while cumc_run enqueues steps, else null
+    unsigned long long *dt_host = nullptr, *dt_pub = nullptr;
     unsigned long long *red = nullptr;  // reduction slots
     double *Ub = nullptr;               // third conserved buffer (stage 2 output)
     bool dt_valid = false;              // dt_dev[1] holds finddt of the current state
@@ -157,7 +160,7 @@ void batch_after_run(cumc_batch *b, int nsteps);
 // ghost passes + torus clamp on the FP64 primitive planes (defined in cumc.hip) and on the
 // mixed form's FP32 planes (cumc_mixed.hip)
 void launch_ghost(cumc_ctx *ctx);
-void launch_ghost32(cumc_ctx *ctx, double *dtnext);
+void launch_ghost32(cumc_ctx *ctx, int st);
 
 // ------------------------------------------------------------------------------------------
 // Segment length of the pencil walks.  A walk of sl faces takes about sl + 1.3 face times (warm-up
@@ -389,7 +392,7 @@ static inline View make_view(const cumc_ctx *ctx, bool col)
 }
 
 // ghost fill of the FP64 primitive planes of a view (defined in cumc.hip)
-void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F, double *dtnext);
+void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F, int st);
 // whether the next step runs in the z-collapsed view (enters it when allowed and the z ghost
 // planes check out), and the return of a collapsed state to the full layout (cumc.hip)
 bool zcollapse_begin(cumc_ctx *ctx);
@@ -419,10 +422,10 @@ void stage_l(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, double *Ub, int st
     mark(ctx, -1);
     mark(ctx, KC_GHOST);
     if constexpr (sizeof(R) == 4) {
-        launch_ghost32(ctx, st == 2 ? ctx->dt_dev + 1 : nullptr);
+        launch_ghost32(ctx, st);
         ctx->p64_stale = true;
     } else {
-        launch_ghost_l(ctx, L, F, st == 2 ? ctx->dt_dev + 1 : nullptr);
+        launch_ghost_l(ctx, L, F, st);
     }
     mark(ctx, -1);
 }

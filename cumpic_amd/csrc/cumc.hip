@@ -173,6 +173,7 @@ extern "C" int cumc_destroy(cumc_ctx *ctx)
     hipFree(ctx->pool);
     hipFree(ctx->fluxpool);
     hipFree(ctx->dt_dev);
+    if (ctx->dt_host) hipHostFree(ctx->dt_host);
     hipFree(ctx->red);
     for (int a = 0; a < 3; a++) {
         hipFree(ctx->tab[a]);
@@ -402,14 +403,14 @@ extern "C" int cumc_download_noalloc(cumc_ctx *ctx, double *prim, double *eps, d
 // ---------------------------------------------------------------------------------------------
 // launch helpers
 // ---------------------------------------------------------------------------------------------
-void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F, double *dtnext)
+void launch_ghost_l(cumc_ctx *ctx, const Lay &L, const Fields<double> &F, int st)
 {
     hipLaunchKernelGGL(k_ghost<double>, dim3(nblk(ghost_threads(L), 256)), dim3(256), 0, ctx->stream, L, F.P, F.EPS, F.BC,
-                       ctx->M, dtnext);
+                       ctx->M, ctx->dt_dev, st, ctx->dt_pub);
     if (!L.zc1) ctx->zfresh = true;
 }
 
-void launch_ghost(cumc_ctx *ctx) { launch_ghost_l(ctx, ctx->L, ctx->F64, nullptr); }
+void launch_ghost(cumc_ctx *ctx) { launch_ghost_l(ctx, ctx->L, ctx->F64, 0); }
 
 // Enters the z-collapsed view when the context allows it and its state is a full-layout state
 // whose z ghost planes the last ghost fill wrote (zfresh) and whose two periodic B_z faces agree.
@@ -576,6 +577,13 @@ static void enqueue_finddt(cumc_ctx *ctx)
     ctx->dt_valid = true;
 }
 
+static int check_dt(cumc_ctx *ctx, double dt)
+{
+    if (!std::isfinite(dt) || !(dt > 0.0) || dt >= 1.0e10)
+        return fail(ctx, CUMC_ENONFINITE, "finddt produced a non-finite step (state has NaN/Inf)");
+    return CUMC_OK;
+}
+
 // dt of the current state into dt_dev[0] (and *dt): the value the last stage 3 left in
 // dt_dev[1] when the state has not changed since, else a finddt launch
 static int finddt_to_current(cumc_ctx *ctx, double *dt)
@@ -591,9 +599,31 @@ static int finddt_to_current(cumc_ctx *ctx, double *dt)
     HIPCHK(ctx, hipMemcpyAsync(dt, ctx->dt_dev + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     collect(ctx);
-    if (!std::isfinite(*dt) || !(*dt > 0.0) || *dt >= 1.0e10)
-        return fail(ctx, CUMC_ENONFINITE, "finddt produced a non-finite step (state has NaN/Inf)");
-    return CUMC_OK;
+    return check_dt(ctx, *dt);
+}
+
+// The same for the step that cumc_run enqueued last, whose ghost fill writes dt to the host's slot
+// (k_ghost).  The slot is watched, the stream asked now and then: a stream that has ended without the
+// slot written (a launch that failed) is left to finddt_to_current.
+constexpr unsigned long long DT_UNSET = ~0ull;
+static int finddt_published(cumc_ctx *ctx, double *dt)
+{
+    unsigned long long bits = DT_UNSET;
+    hipError_t e = hipErrorNotReady;
+    while (e == hipErrorNotReady) {
+        for (int i = 0; i < 4096 && bits == DT_UNSET; i++) {
+            __builtin_ia32_pause();
+            bits = __atomic_load_n(ctx->dt_host, __ATOMIC_ACQUIRE);
+        }
+        if (bits != DT_UNSET) break;
+        e = hipStreamQuery(ctx->stream);
+        if (e == hipErrorNotReady) (void)hipGetLastError();
+    }
+    if (bits == DT_UNSET) return finddt_to_current(ctx, dt);
+    std::memcpy(dt, &bits, sizeof bits);
+    const int r = check_dt(ctx, *dt);
+    if (r) HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return r;
 }
 
 extern "C" int cumc_finddt(cumc_ctx *ctx, double *dt)
@@ -631,16 +661,28 @@ extern "C" int cumc_run(cumc_ctx *ctx, int max_steps, double total_time, double 
     bool graphs = max_steps >= 8 && !ctx->prof;
     StepGraphs sg(ctx->stream);
     int par = 0;  // conserved-buffer parity of the step within this call
+    // dt from step to step through the host's slot (profiling collects its events at each step's wait)
+    struct Publishing {
+        cumc_ctx *c;
+        ~Publishing() { c->dt_pub = nullptr; }
+    } publishing{ctx};
+    if (!ctx->prof && !ctx->dt_host &&
+        hipHostMalloc((void **)&ctx->dt_host, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+        ctx->dt_host = nullptr;
+    if (ctx->prof || !ctx->dt_host || hipHostGetDevicePointer((void **)&ctx->dt_pub, ctx->dt_host, 0) != hipSuccess)
+        ctx->dt_pub = nullptr;
+    (void)hipGetLastError();  // (without the slot the steps go by copies)
     HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     while (global_time < total_time && n < max_steps) {
         double dt;
-        int r = finddt_to_current(ctx, &dt);
+        int r = ctx->dt_pub && n > 0 ? finddt_published(ctx, &dt) : finddt_to_current(ctx, &dt);
         if (r) { *time = global_time; if (steps_done) *steps_done = n; return r; }
         if (global_time + dt > total_time) {
             dt = total_time - global_time;
             HIPCHK(ctx, hipMemcpyAsync(ctx->dt_dev, &dt, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
             HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         }
+        if (ctx->dt_pub) __atomic_store_n(ctx->dt_host, DT_UNSET, __ATOMIC_RELEASE);
         if (graphs) {
             const bool zc = ctx->cfg.precision != CUMC_MIXED && zcollapse_begin(ctx);
             hipGraphExec_t &ex = sg.ex[par][zc ? 1 : 0];

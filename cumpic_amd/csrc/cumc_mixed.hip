@@ -8,12 +8,12 @@
 void stage_mixed(cumc_ctx *ctx, int st, bool comb) { stage<float>(ctx, ctx->F32, st, comb); }
 
 // the reference's ghost passes (and torus inflow clamps) on the FP32 primitive planes
-void launch_ghost32(cumc_ctx *ctx, double *dtnext)
+void launch_ghost32(cumc_ctx *ctx, int st)
 {
     const Lay &L = ctx->L;
     const Fields<float> &G = ctx->F32;
     hipLaunchKernelGGL(k_ghost<float>, dim3(nblk(ghost_threads(L), 256)), dim3(256), 0, ctx->stream, L, G.P32, G.EPS32,
-                       G.BC32, ctx->M, dtnext);
+                       G.BC32, ctx->M, ctx->dt_dev, st, ctx->dt_pub);
 }
 
 void fluxes_mixed(cumc_ctx *ctx, int dir, double *aos_tmp)
