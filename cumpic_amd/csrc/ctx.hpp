@@ -28,8 +28,8 @@ struct cumc_ctx {
     double *tab[3] = {nullptr, nullptr, nullptr};
     float *tabf[3] = {nullptr, nullptr, nullptr};
     double *dt_dev = nullptr;           // [0] dt of the current step, [1] dt found by stage 3
-    // pinned word through which a run's steps hand the next dt to the host (finddt_published);
-    // dt_pub is its device address while cumc_run enqueues steps, else null
+    // pinned word through which a call's steps hand the next dt to the host (DtHandOn); dt_pub
+    // is its device address while one lives, else null
     unsigned long long *dt_host = nullptr, *dt_pub = nullptr;
     unsigned long long *red = nullptr;  // reduction slots
     double *Ub = nullptr;               // third conserved buffer (stage 2 output)
@@ -131,6 +131,18 @@ static inline void swap_u(cumc_ctx *ctx)
     ctx->F32.U0 = ctx->F64.U0;
     ctx->F32.U1 = ctx->F64.U1;
 }
+
+// The time step handed from step to step of one call through the context's pinned word (k_ghost;
+// defined in cumc.hip).  While it lives, stage-3 ghost fills make the step they find the current one and
+// publish it.  Without the word (off, profiling, no memory) next() is finddt as a call by itself makes it.
+struct DtHandOn {
+    cumc_ctx *ctx;
+    bool pending = false;  // a step that will publish is enqueued
+    DtHandOn(cumc_ctx *c, bool on);
+    ~DtHandOn() { ctx->dt_pub = nullptr; }
+    int next(double *dt);  // dt of the current state, in dt_dev[0] too
+    void enqueue();        // ahead of a step's launches
+};
 
 // frees the reverse-mode record (defined in cumc_adjoint.hip)
 void tape_release(cumc_ctx *ctx);

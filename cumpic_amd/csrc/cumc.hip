@@ -602,12 +602,31 @@ static int finddt_to_current(cumc_ctx *ctx, double *dt)
     return check_dt(ctx, *dt);
 }
 
-// The same for the step that cumc_run enqueued last, whose ghost fill writes dt to the host's slot
-// (k_ghost).  The slot is watched, the stream asked now and then: a stream that has ended without the
-// slot written (a launch that failed) is left to finddt_to_current.
 constexpr unsigned long long DT_UNSET = ~0ull;
-static int finddt_published(cumc_ctx *ctx, double *dt)
+DtHandOn::DtHandOn(cumc_ctx *c, bool on) : ctx(c)
 {
+    ctx->dt_pub = nullptr;
+    if (!on || ctx->prof) return;  // (profiling collects its events at each step's wait)
+    if (!ctx->dt_host && hipHostMalloc((void **)&ctx->dt_host, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+        ctx->dt_host = nullptr;
+    if (!ctx->dt_host || hipHostGetDevicePointer((void **)&ctx->dt_pub, ctx->dt_host, 0) != hipSuccess) {
+        ctx->dt_pub = nullptr;
+        (void)hipGetLastError();
+    }
+}
+void DtHandOn::enqueue()
+{
+    if (!ctx->dt_pub) return;
+    __atomic_store_n(ctx->dt_host, DT_UNSET, __ATOMIC_RELEASE);
+    pending = true;
+}
+// The first step of a call waits for the stream (nothing enqueued earlier can publish after that); the
+// later ones watch the word and ask the stream now and then: a stream that has ended without the word
+// written (a launch that failed) is left to finddt_to_current.
+int DtHandOn::next(double *dt)
+{
+    if (!pending) return finddt_to_current(ctx, dt);
+    pending = false;
     unsigned long long bits = DT_UNSET;
     hipError_t e = hipErrorNotReady;
     while (e == hipErrorNotReady) {
@@ -661,28 +680,18 @@ extern "C" int cumc_run(cumc_ctx *ctx, int max_steps, double total_time, double 
     bool graphs = max_steps >= 8 && !ctx->prof;
     StepGraphs sg(ctx->stream);
     int par = 0;  // conserved-buffer parity of the step within this call
-    // dt from step to step through the host's slot (profiling collects its events at each step's wait)
-    struct Publishing {
-        cumc_ctx *c;
-        ~Publishing() { c->dt_pub = nullptr; }
-    } publishing{ctx};
-    if (!ctx->prof && !ctx->dt_host &&
-        hipHostMalloc((void **)&ctx->dt_host, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-        ctx->dt_host = nullptr;
-    if (ctx->prof || !ctx->dt_host || hipHostGetDevicePointer((void **)&ctx->dt_pub, ctx->dt_host, 0) != hipSuccess)
-        ctx->dt_pub = nullptr;
-    (void)hipGetLastError();  // (without the slot the steps go by copies)
+    DtHandOn hand_on(ctx, true);
     HIPCHK(ctx, hipEventRecord(ctx->ev0, ctx->stream));
     while (global_time < total_time && n < max_steps) {
         double dt;
-        int r = ctx->dt_pub && n > 0 ? finddt_published(ctx, &dt) : finddt_to_current(ctx, &dt);
+        int r = hand_on.next(&dt);
         if (r) { *time = global_time; if (steps_done) *steps_done = n; return r; }
         if (global_time + dt > total_time) {
             dt = total_time - global_time;
             HIPCHK(ctx, hipMemcpyAsync(ctx->dt_dev, &dt, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
             HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         }
-        if (ctx->dt_pub) __atomic_store_n(ctx->dt_host, DT_UNSET, __ATOMIC_RELEASE);
+        hand_on.enqueue();
         if (graphs) {
             const bool zc = ctx->cfg.precision != CUMC_MIXED && zcollapse_begin(ctx);
             hipGraphExec_t &ex = sg.ex[par][zc ? 1 : 0];
