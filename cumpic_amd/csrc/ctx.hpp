@@ -45,8 +45,8 @@ struct cumc_ctx {
     bool zbad = false;   // the entry check found unequal periodic B_z faces (until the next upload)
     bool ztape = false;  // a reverse-mode record holds full-layout states: no collapsed steps
     struct cumc_tape *tape = nullptr;  // reverse-mode record (cumc_adjoint.hip)
-    int seg = 24;    // target faces per pencil segment of the y / z sweeps
-    int zchunk = 4;  // planes per column tile of the EMF and stage-tail kernels
+    int seg = 24;    // most faces per pencil segment of the y / z sweeps
+    int zchunk = 4;  // most planes per column tile of the EMF and stage-tail kernels
     int tile_w = 0;   // column tile width of those kernels (0: flattened rows; see col_of)
     double last_ms = 0.0;
     std::string err;

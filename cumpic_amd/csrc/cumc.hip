@@ -495,7 +495,7 @@ static void enqueue_step(cumc_ctx *ctx)
 
 // cumc_run's steps as hipGraphs: one graph per conserved-buffer parity and view, captured on
 // first use within the call and destroyed at its end, so no graph outlives the buffers, view and
-// launch shapes it was captured with.  On small grids the ~24 launches of a step cost more than
+// launch shapes it was captured with.  On small grids the 12 launches of a step cost more than
 // their kernels.  The view is settled (zcollapse_begin, which may synchronise the stream) before
 // any capture; a capture that fails leaves the step to direct launches.
 struct StepGraphs {
@@ -607,7 +607,8 @@ DtHandOn::DtHandOn(cumc_ctx *c, bool on) : ctx(c)
 {
     ctx->dt_pub = nullptr;
     if (!on || ctx->prof) return;  // (profiling collects its events at each step's wait)
-    if (!ctx->dt_host && hipHostMalloc((void **)&ctx->dt_host, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+    if (!ctx->dt_host && hipHostMalloc((void **)&ctx->dt_host, 64,
+                                       hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
         ctx->dt_host = nullptr;
     if (!ctx->dt_host || hipHostGetDevicePointer((void **)&ctx->dt_pub, ctx->dt_host, 0) != hipSuccess) {
         ctx->dt_pub = nullptr;

@@ -143,8 +143,8 @@ const char *cumc_last_error(cumc_ctx *ctx);
 enum { CUMC_PH_FLUX_X = 0, CUMC_PH_FLUX_Y, CUMC_PH_FLUX_Z, CUMC_PH_ECORN, CUMC_PH_TAIL, CUMC_PH_GHOST,
        CUMC_PH_FINDDT, CUMC_PH_N };
 typedef struct cumc_tuning {
-    int seg;                 /* target faces per pencil segment of the y and z sweeps */
-    int zchunk;              /* planes per column tile of the EMF and stage-tail kernels */
+    int seg;                 /* most faces per pencil segment of the y and z sweeps */
+    int zchunk;              /* most planes per column tile of the EMF and stage-tail kernels */
     int blocks[CUMC_PH_N];   /* batch only: persistent workgroups per phase, 0 = one per tile */
     int tile_w;              /* column tile of the EMF / stage-tail kernels: 0 = flattened rows of 256
                                 cells, or 32 / 64 / 128 = tile_w x (256 / tile_w) columns */
