@@ -174,6 +174,11 @@ __device__ inline void flux_x_wave(const Lay &L, const Fields<R> &F, const Tabs 
     const int j = jj - 2;
     const bool active = lane >= 2 && lane <= 60 && inr && k <= L.ny + 1 && j >= 0 && j <= L.nx;
     const int jc = j < -2 ? -2 : (j > L.nx + 3 ? L.nx + 3 : j);
+#ifdef CUMC_BRANCH_SIG
+    // decisions on cells no face of the wavefront takes (ends of the stencil, row padding) are not recorded
+    const bool needed = lane >= 2 && lane <= 61 && inr && k <= L.ny + 1 && j >= 0 && j <= L.nx + 1;
+    const unsigned long long before = br_slot[threadIdx.x];
+#endif
 
     const unsigned gu = (unsigned)g;
     const long ps = L.ps;
@@ -209,6 +214,9 @@ __device__ inline void flux_x_wave(const Lay &L, const Fields<R> &F, const Tabs 
     FaceState<R> sr{vr[0], vr[1], vr[2], vr[3], vr[4], bn, vr[5], vr[6]};
     R fl[7];
     riemann_face<1, R, SOLVER>(R(M.ggas), sl, sr, fl);
+#ifdef CUMC_BRANCH_SIG
+    if (!needed) br_slot[threadIdx.x] = before;
+#endif
     if (active) {
         R *o = F.F[0];
 #pragma unroll
