@@ -327,6 +327,14 @@ __device__ inline void flux_ylane_tile(const Lay &L, const Fields<R> &F, const T
 // FP32: two, whose neighbouring rows meet in one compute unit's cache (192^3 mixed 126 against 128 us).
 template <typename R>
 constexpr int walk_block() { return sizeof(R) == 8 ? 64 : 128; }
+// Wavefronts per SIMD that the registers of the FP64 sweeps are capped for.  Three (168 VGPRs) suit HLL
+// and LF, and HLLC behind TVD (2 to 8 spilled registers there cost less than the third wavefront gives:
+// 160^3 3054 us a step against 3133 with two).  HLLD needs up to 224 VGPRs and HLLC behind PPM or WENO5 up
+// to 194: at three they spilled 80 to 189 and 15 to 34 registers, two wavefronts keep all of them.  Per step,
+// three against two: PPM + HLLD 48^3 251 -> 199 us, 96^3 1376 -> 808, 160^3 5774 -> 3314; TVD + HLLD 160^3
+// 5365 -> 3298; PPM + HLLC 96^3 890 -> 767, 160^3 3525 -> 3130.
+template <int RECON, int SOLVER>
+constexpr int sweep_waves() { return SOLVER == 4 || (SOLVER == 3 && RECON >= 4) ? 2 : 3; }
 // One walk_block-thread tile: bx covers px*(nt+2) pencils, segment by of seglen faces along DIR.
 template <typename R, int DIR, int RECON, int SOLVER = 2>
 __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Tabs &tb, const Model &M, int seglen,
@@ -501,7 +509,7 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
 }
 
 template <typename R, int DIR, int RECON, int SOLVER>
-__global__ __launch_bounds__(walk_block<R>(), sizeof(R) == 8 ? 3 : 1) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
+__global__ __launch_bounds__(walk_block<R>(), (sizeof(R) == 8 ? sweep_waves<RECON, SOLVER>() : 1)) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
 {
     flux_walk_tile<R, DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
 }
@@ -520,7 +528,7 @@ struct SweepGrid {
     int x_waves;          // x wavefronts per plane
 };
 template <int RECON, int SOLVER>
-__global__ __launch_bounds__(64, 3) void k_flux_xyz(Lay L, Fields<double> F, Tabs tb, Model M, SweepGrid G)
+__global__ __launch_bounds__(64, (sweep_waves<RECON, SOLVER>())) void k_flux_xyz(Lay L, Fields<double> F, Tabs tb, Model M, SweepGrid G)
 {
     int b = (int)blockIdx.x;
     if (b < G.y_n) {
