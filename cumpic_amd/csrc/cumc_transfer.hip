@@ -44,6 +44,7 @@ bool make_unit(int device, Unit &u)
         hipMalloc(&u.dev, STAGE_BYTES) == hipSuccess && hipHostMalloc(&u.pin, STAGE_BYTES, hipHostMallocDefault) == hipSuccess)
         return true;
     free_unit(u);
+    (void)hipGetLastError();  // (else the next launch's check on this thread reports it)
     return false;
 }
 
@@ -137,17 +138,19 @@ hipError_t run_piece(const Lay &L, const Piece &p, bool out, const Unit &u)
     hipError_t e;
     if (out) {
         hipLaunchKernelGGL(k_piece_to_aos, grid, dim3(256), 0, u.stream, L, (const double *)p.a.soa, p.a.nv, p.c0, p.n, u.dev);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if ((e = hipMemcpyAsync(u.pin, u.dev, bytes, hipMemcpyDeviceToHost, u.stream)) != hipSuccess) return e;
-        if ((e = hipStreamSynchronize(u.stream)) != hipSuccess) return e;
-        std::memcpy(host, u.pin, bytes);
-        return hipSuccess;
+        if ((e = hipGetLastError()) == hipSuccess) e = hipMemcpyAsync(u.pin, u.dev, bytes, hipMemcpyDeviceToHost, u.stream);
+    } else {
+        std::memcpy(u.pin, host, bytes);
+        if ((e = hipMemcpyAsync(u.dev, u.pin, bytes, hipMemcpyHostToDevice, u.stream)) == hipSuccess) {
+            hipLaunchKernelGGL(k_piece_to_soa, grid, dim3(256), 0, u.stream, L, p.a.soa, p.a.nv, p.c0, p.n, (const double *)u.dev);
+            e = hipGetLastError();
+        }
     }
-    std::memcpy(u.pin, host, bytes);
-    if ((e = hipMemcpyAsync(u.dev, u.pin, bytes, hipMemcpyHostToDevice, u.stream)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_piece_to_soa, grid, dim3(256), 0, u.stream, L, p.a.soa, p.a.nv, p.c0, p.n, (const double *)u.dev);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    return hipStreamSynchronize(u.stream);
+    // (waits after an error too: the unit goes back for the next transfer to use)
+    const hipError_t w = hipStreamSynchronize(u.stream);
+    if (e == hipSuccess) e = w;
+    if (e == hipSuccess && out) std::memcpy(host, u.pin, bytes);
+    return e;
 }
 
 int transfer(cumc_ctx *ctx, const XferArray *a, int n, bool out)
