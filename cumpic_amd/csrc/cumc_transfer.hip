@@ -13,84 +13,143 @@
 
 namespace {
 
-constexpr size_t STAGE_BYTES = size_t(2) << 20;  // one piece; a unit holds it on the device and pinned on the host
-constexpr int MAX_UNITS = 8;                     // per device: at most 16 MiB of either kind of memory
-constexpr size_t BYTES_PER_UNIT = size_t(2) << 20;  // a transfer takes one more unit per this much
+constexpr size_t UNIT_BYTES = size_t(2) << 20;  // of device memory and of pinned host memory, per unit
+constexpr int MAX_UNITS = 8;                    // per device: at most 16 MiB of either kind of memory
+constexpr int MAX_DEVICES = 64;
+// A transfer takes one more unit per this much.  Below it a second thread costs more than it saves: download of
+// 22^3 (2.1 MB) 144 us on one, 164 on two; of 36^3 267 on two, 312 on three.
+constexpr size_t BYTES_PER_UNIT = size_t(3) << 20;
+// A stream costs about 0.75 ms to make and destroy, in which one unit moves about this much.
+constexpr double STREAM_BYTES = double(4 << 20);
 
 struct Unit {
     int device = 0;
-    hipStream_t stream = nullptr;
     double *dev = nullptr;
     double *pin = nullptr;
+};
+// Units made together are one allocation of either kind: each costs 0.3 to 0.5 ms to make and as much to
+// free, whatever its size.
+struct Block {
+    int device = 0;
+    void *dev = nullptr, *pin = nullptr;
+};
+struct Device {
+    int units = 0, streams = 0;  // made, idle or in use
+    double owed = 0.0;           // bytes' worth of time that one more stream would have saved so far
+    std::vector<hipStream_t> idle;
 };
 
 std::mutex g_mu;
 std::condition_variable g_cv;
-std::vector<Unit> g_free;   // idle units of every device
-int g_made[64] = {0};       // units made per device, idle or in use
+std::vector<Unit> g_free;  // idle units of every device
+std::vector<Block> g_blocks;
+Device g_dev[MAX_DEVICES];
 int g_users = 0;
 
-void free_unit(Unit &u)
+void free_block(Block &b)
 {
-    if (u.stream) (void)hipStreamDestroy(u.stream);
-    (void)hipFree(u.dev);
-    (void)hipHostFree(u.pin);
+    (void)hipFree(b.dev);
+    (void)hipHostFree(b.pin);
 }
 
-bool make_unit(int device, Unit &u)
+// n more units of the current device among the idle ones
+bool make_units(int device, int n)
 {
-    u.device = device;
-    if (hipStreamCreateWithFlags(&u.stream, hipStreamNonBlocking) == hipSuccess &&
-        hipMalloc(&u.dev, STAGE_BYTES) == hipSuccess && hipHostMalloc(&u.pin, STAGE_BYTES, hipHostMallocDefault) == hipSuccess)
-        return true;
-    free_unit(u);
-    (void)hipGetLastError();  // (else the next launch's check on this thread reports it)
-    return false;
-}
-
-// Between 1 and `want` units of the current device.  A call waits only while other transfers hold all
-// of them; none are held while waiting, so every waiter is served in the end.  Empty: out of memory.
-std::vector<Unit> acquire(int device, int want)
-{
-    std::vector<Unit> got;
-    got.reserve(want);
-    std::unique_lock<std::mutex> lock(g_mu);
-    for (;;) {
-        for (size_t i = 0; i < g_free.size() && (int)got.size() < want;) {
-            if (g_free[i].device == device) {
-                got.push_back(g_free[i]);
-                g_free.erase(g_free.begin() + (long)i);
-            } else {
-                i++;
-            }
-        }
-        while ((int)got.size() < want && g_made[device] < MAX_UNITS) {
-            Unit u;
-            if (!make_unit(device, u)) break;
-            g_made[device]++;
-            got.push_back(u);
-        }
-        if (!got.empty() || g_made[device] == 0) return got;
-        g_cv.wait(lock);
+    g_blocks.reserve(g_blocks.size() + 1);
+    g_free.reserve(g_free.size() + MAX_UNITS);
+    Block b;
+    b.device = device;
+    if (hipMalloc(&b.dev, n * UNIT_BYTES) != hipSuccess || hipHostMalloc(&b.pin, n * UNIT_BYTES, hipHostMallocDefault) != hipSuccess) {
+        free_block(b);
+        (void)hipGetLastError();  // (else the next launch's check on this thread reports it)
+        return false;
     }
+    g_blocks.push_back(b);
+    for (int i = 0; i < n; i++) {
+        Unit u;
+        u.device = device;
+        u.dev = (double *)((char *)b.dev + i * UNIT_BYTES);
+        u.pin = (double *)((char *)b.pin + i * UNIT_BYTES);
+        g_free.push_back(u);
+    }
+    g_dev[device].units += n;
+    return true;
 }
 
-void give_back(std::vector<Unit> &units)
-{
+// The units and streams of one transfer: a unit each for as many host threads, the first on the context's
+// own stream and the others on one of these.
+struct Lease {
+    int device = 0;
+    std::vector<Unit> units;
+    std::vector<hipStream_t> streams;
+
+    // At least one unit of the current device and at most `want`, for a transfer of `bytes`.  A call waits
+    // only while other transfers hold all of them; none are held while waiting, so every waiter is served
+    // in the end.  No units: out of memory.
+    // One more unit at a time is worth a stream once the time it saves, here or added up over the transfers
+    // so far, is the time the stream takes to make and destroy: a process that opens a context, moves little
+    // and closes it again must not pay for eight.  64^3 opened, uploaded, stepped four times, downloaded and
+    // closed: 15.5 ms with eight units made one by one at the first transfer, 5.5 ms so; repeated transfers
+    // have as many units as before after the first few.
+    void take(int dev, int want, double bytes)
     {
-        std::lock_guard<std::mutex> lock(g_mu);
-        for (Unit &u : units) {
-            if (g_users > 0) {
-                g_free.push_back(u);
-            } else {
-                g_made[u.device]--;
-                free_unit(u);
+        device = dev;
+        Device &d = g_dev[dev];
+        units.reserve(want);
+        streams.reserve(want);
+        std::unique_lock<std::mutex> lock(g_mu);
+        d.idle.reserve(MAX_UNITS);
+        for (;;) {
+            int free = 0;
+            for (const Unit &u : g_free) free += u.device == dev;
+            const int room = MAX_UNITS - d.units, lack = want - free < room ? want - free : room;
+            // (one unit alone where there is no memory for all)
+            if (lack > 0 && !make_units(dev, lack) && free == 0 && lack > 1) make_units(dev, 1);
+            for (size_t i = 0; i < g_free.size() && (int)units.size() < want;) {
+                if (g_free[i].device == dev) {
+                    units.push_back(g_free[i]);
+                    g_free.erase(g_free.begin() + (long)i);
+                } else {
+                    i++;
+                }
             }
+            if (!units.empty() || d.units == 0) break;
+            g_cv.wait(lock);
+        }
+        while (streams.size() + 1 < units.size()) {
+            hipStream_t s = nullptr;
+            if (!d.idle.empty()) {
+                s = d.idle.back();
+                d.idle.pop_back();
+            } else {
+                const double k = (double)streams.size() + 1.0;
+                d.owed += bytes / (k * (k + 1.0));
+                if (d.streams >= MAX_UNITS - 1 || d.owed < STREAM_BYTES) break;
+                if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
+                    (void)hipGetLastError();
+                    break;
+                }
+                d.streams++;
+                d.owed = 0.0;
+            }
+            streams.push_back(s);
+        }
+        while (units.size() > streams.size() + 1) {
+            g_free.push_back(units.back());
+            units.pop_back();
         }
     }
-    units.clear();
-    g_cv.notify_all();
-}
+    ~Lease()
+    {
+        {
+            std::lock_guard<std::mutex> lock(g_mu);
+            // (room for all was reserved as they were made)
+            for (Unit &u : units) g_free.push_back(u);
+            for (hipStream_t s : streams) g_dev[device].idle.push_back(s);
+        }
+        g_cv.notify_all();
+    }
+};
 
 // cells [c0, c0 + n) of the box (in the caller's cell order) between the planes and a piece
 __global__ __launch_bounds__(256) void k_piece_to_aos(Lay L, const double *__restrict__ soa, int nv, long c0, int n,
@@ -130,28 +189,71 @@ struct Piece {
     int n;
 };
 
-hipError_t run_piece(const Lay &L, const Piece &p, bool out, const Unit &u)
-{
-    const size_t bytes = (size_t)p.n * p.a.nv * sizeof(double);
-    double *host = p.a.host + p.c0 * p.a.nv;
-    const dim3 grid(nblk(p.n, 256));
-    hipError_t e;
-    if (out) {
-        hipLaunchKernelGGL(k_piece_to_aos, grid, dim3(256), 0, u.stream, L, (const double *)p.a.soa, p.a.nv, p.c0, p.n, u.dev);
-        if ((e = hipGetLastError()) == hipSuccess) e = hipMemcpyAsync(u.pin, u.dev, bytes, hipMemcpyDeviceToHost, u.stream);
-    } else {
-        std::memcpy(u.pin, host, bytes);
-        if ((e = hipMemcpyAsync(u.dev, u.pin, bytes, hipMemcpyHostToDevice, u.stream)) == hipSuccess) {
-            hipLaunchKernelGGL(k_piece_to_soa, grid, dim3(256), 0, u.stream, L, p.a.soa, p.a.nv, p.c0, p.n, (const double *)u.dev);
-            e = hipGetLastError();
-        }
+// One thread's pieces through one unit and one stream.  They are queued until the unit is full and waited
+// for together, conversions next to each other and copies next to each other (going from one engine to the
+// other and back costs about 15 us): a box that fits into a unit costs one wait.
+struct Worker {
+    const Lay &L;
+    bool out;
+    const Unit &u;
+    hipStream_t st;
+    size_t used = 0;  // bytes of the unit that queued pieces hold
+    std::vector<std::pair<const Piece *, size_t>> queued;
+
+    static size_t bytes_of(const Piece &p) { return (size_t)p.n * p.a.nv * sizeof(double); }
+    double *at(double *base, size_t off) const { return base + off / sizeof(double); }
+    hipError_t convert(const Piece &p, size_t off)
+    {
+        const dim3 grid(nblk(p.n, 256));
+        double *dev = at(u.dev, off);
+        if (out)
+            hipLaunchKernelGGL(k_piece_to_aos, grid, dim3(256), 0, st, L, (const double *)p.a.soa, p.a.nv, p.c0, p.n, dev);
+        else
+            hipLaunchKernelGGL(k_piece_to_soa, grid, dim3(256), 0, st, L, p.a.soa, p.a.nv, p.c0, p.n, (const double *)dev);
+        return hipGetLastError();
     }
-    // (waits after an error too: the unit goes back for the next transfer to use)
-    const hipError_t w = hipStreamSynchronize(u.stream);
-    if (e == hipSuccess) e = w;
-    if (e == hipSuccess && out) std::memcpy(host, u.pin, bytes);
-    return e;
-}
+    // the other half of what is queued, and the wait for all of it
+    hipError_t flush()
+    {
+        hipError_t e = hipSuccess;
+        if (out && used) e = hipMemcpyAsync(u.pin, u.dev, used, hipMemcpyDeviceToHost, st);
+        for (const auto &[p, off] : queued)
+            if (!out && e == hipSuccess) e = convert(*p, off);
+        const hipError_t w = hipStreamSynchronize(st);
+        if (e == hipSuccess) e = w;
+        for (const auto &[p, off] : queued)
+            if (out && e == hipSuccess) std::memcpy(p->a.host + p->c0 * p->a.nv, at(u.pin, off), bytes_of(*p));
+        queued.clear();
+        used = 0;
+        return e;
+    }
+    hipError_t put(const Piece &p)
+    {
+        const size_t bytes = bytes_of(p);
+        hipError_t e = used + bytes > UNIT_BYTES ? flush() : hipSuccess;
+        if (e != hipSuccess) return e;
+        const size_t off = used;
+        if (out) {
+            e = convert(p, off);
+        } else {
+            std::memcpy(at(u.pin, off), p.a.host + p.c0 * p.a.nv, bytes);
+            e = hipMemcpyAsync(at(u.dev, off), at(u.pin, off), bytes, hipMemcpyHostToDevice, st);
+        }
+        queued.emplace_back(&p, off);
+        used += (bytes + 255) / 256 * 256 < UNIT_BYTES - used ? (bytes + 255) / 256 * 256 : UNIT_BYTES - used;
+        return e;
+    }
+    // shares the pieces with the other workers; leaves nothing queued, after an error either (the unit goes
+    // back for the next transfer to use)
+    void run(const std::vector<Piece> &pieces, std::atomic<size_t> &next, std::atomic<int> &err)
+    {
+        hipError_t e = hipSuccess;
+        for (size_t i = next++; i < pieces.size() && e == hipSuccess && err == (int)hipSuccess; i = next++) e = put(pieces[i]);
+        if (e == hipSuccess) e = flush();
+        else (void)hipStreamSynchronize(st);
+        if (e != hipSuccess) err = (int)e;
+    }
+};
 
 int transfer(cumc_ctx *ctx, const XferArray *a, int n, bool out)
 {
@@ -161,42 +263,45 @@ int transfer(cumc_ctx *ctx, const XferArray *a, int n, bool out)
     const OnDevice here(ctx->device);
     HIPCHK(ctx, here.e);
     const int device = ctx->device;
-    if (device < 0 || device >= 64) return fail(ctx, CUMC_EINVAL, "device index out of range");
+    if (device < 0 || device >= MAX_DEVICES) return fail(ctx, CUMC_EINVAL, "device index out of range");
     try {
-        std::vector<Piece> pieces;
         size_t bytes = 0;
+        for (int i = 0; i < n; i++) bytes += (size_t)ncell * a[i].nv * sizeof(double);
+        const int want = bytes / BYTES_PER_UNIT + 1 > MAX_UNITS ? MAX_UNITS : (int)(bytes / BYTES_PER_UNIT + 1);
+        Lease lease;
+        lease.take(device, want, (double)bytes);
+        if (lease.units.empty()) return fail(ctx, CUMC_ENOMEM, "transfer staging");
+        // pieces of at most a unit for several threads, of equal size and as many for one as for another; of a
+        // third of a unit for one thread, so that copying one overlaps the engine's work on the one before
+        const size_t k = lease.units.size(), rounds = bytes / (k * UNIT_BYTES) + 1;
+        const size_t share = k > 1 ? bytes / (k * rounds) + 4096 : UNIT_BYTES / 3;
+        const size_t most = share < UNIT_BYTES ? share : UNIT_BYTES;
+        std::vector<Piece> pieces;
         for (int i = 0; i < n; i++) {
-            const long per = (long)(STAGE_BYTES / sizeof(double)) / a[i].nv;
+            const long per = (long)(most / sizeof(double)) / a[i].nv;
             for (long c = 0; c < ncell; c += per) pieces.push_back({a[i], c, (int)(ncell - c < per ? ncell - c : per)});
-            bytes += (size_t)ncell * a[i].nv * sizeof(double);
         }
-        int want = 1 + (int)(bytes / BYTES_PER_UNIT);
-        want = want > MAX_UNITS ? MAX_UNITS : want;
-        std::vector<Unit> units = acquire(device, want);
-        if (units.empty()) return fail(ctx, CUMC_ENOMEM, "transfer staging");
         std::atomic<size_t> next{0};
         std::atomic<int> err{(int)hipSuccess};
-        auto work = [&](const Unit &u) {
-            for (size_t i = next++; i < pieces.size() && err == (int)hipSuccess; i = next++) {
-                const hipError_t e = run_piece(L, pieces[i], out, u);
-                if (e != hipSuccess) err = (int)e;
-            }
-        };
+        std::vector<Worker> workers;
+        for (size_t i = 0; i < k; i++) {
+            workers.push_back(Worker{L, out, lease.units[i], i ? lease.streams[i - 1] : ctx->stream});
+            workers[i].queued.reserve(pieces.size());
+        }
         std::vector<std::thread> threads;
+        threads.reserve(k);
         try {
-            threads.reserve(units.size());
-            for (size_t i = 1; i < units.size(); i++)
+            for (size_t i = 1; i < k; i++)
                 threads.emplace_back([&, i]() {
                     const hipError_t e = hipSetDevice(device);
                     if (e != hipSuccess) err = (int)e;
-                    else work(units[i]);
+                    else workers[i].run(pieces, next, err);
                 });
         } catch (const std::exception &) {
             // no further thread to be had: the ones that run share the pieces
         }
-        work(units[0]);
+        workers[0].run(pieces, next, err);
         for (std::thread &t : threads) t.join();
-        give_back(units);
         const hipError_t e = (hipError_t)err.load();
         if (e != hipSuccess) return fail(ctx, CUMC_EHIP, std::string("transfer: ") + hipGetErrorString(e));
     } catch (const std::exception &x) {
@@ -222,10 +327,14 @@ void staging_release()
     if (--g_users > 0) return;
     int cur = 0;
     const bool back = hipGetDevice(&cur) == hipSuccess;
-    for (Unit &u : g_free) {
-        if (hipSetDevice(u.device) == hipSuccess) free_unit(u);
-        g_made[u.device]--;
-    }
+    for (Block &b : g_blocks)
+        if (hipSetDevice(b.device) == hipSuccess) free_block(b);
+    g_blocks.clear();
     g_free.clear();
+    for (int i = 0; i < MAX_DEVICES; i++) {
+        if (!g_dev[i].idle.empty() && hipSetDevice(i) == hipSuccess)
+            for (hipStream_t st : g_dev[i].idle) (void)hipStreamDestroy(st);
+        g_dev[i] = Device{};
+    }
     if (back) (void)hipSetDevice(cur);
 }

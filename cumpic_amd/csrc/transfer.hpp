@@ -1,12 +1,13 @@
 // transfer.hpp -- host arrays in and out of the device planes.
 //
 // A transfer converts between the caller's AoS arrays (cell-major, nv values per cell) and the SoA
-// planes in pieces of STAGE_BYTES: device staging buffer, pinned host buffer, caller's memory.  A
-// temporary of the array's size on each call cost a hipMalloc and hipFree (which waits for the device)
-// and a copy from or to pageable memory at one thread's page-fault rate; here the staging units are
-// kept, and a large transfer runs several of them at once, one host thread each, so that conversion,
-// copy and the caller's page faults overlap.  Download of 256^3 (1.7 GB) 168 -> 40 ms, of a 400^2 box
-// (111 MB, seven planes) 12.7 -> 3.1 ms, upload of 256^3 (1.3 GB) 58 -> 39 ms.
+// planes in pieces: device staging buffer, pinned host buffer, caller's memory.  A temporary of the array's
+// size on each call cost a hipMalloc and hipFree (which waits for the device) and a copy from or to pageable
+// memory at one thread's page-fault rate; here the staging units (2 MiB of either memory) are kept while
+// there is a context, and a large transfer runs up to eight of them at once, one host thread each, so that
+// conversion, copy and the caller's page faults overlap.  Download of 256^3 (1.7 GB) 166 -> 35 ms, of a 400^2
+// box (111 MB, seven planes) 10.0 -> 2.5 ms, of 24^3 200 -> 185 us; upload of 256^3 (1.3 GB) 43 -> 23 ms, of
+// 24^3 122 -> 120 us.
 #pragma once
 #include "ctx.hpp"
 

@@ -19,14 +19,8 @@ thread_local std::vector<Call> calls;
 long allocs_left = 1L << 40, launches_left = 1L << 40;
 long streams_made = 0, allocs_made = 0, live = 0;
 
-struct Stream;
-struct Event {
-    Stream *on = nullptr;
-    long number = 0;  // position of the last record in its stream
-};
 struct Stream {
     std::deque<std::function<void()>> work;
-    long done = 0, queued = 0;
 };
 std::map<hipStream_t, Stream *> streams;
 
@@ -35,20 +29,6 @@ hipError_t error(hipError_t e)
     last = e;
     return e;
 }
-void push(Stream *s, std::function<void()> f)
-{
-    s->work.push_back(std::move(f));
-    s->queued++;
-}
-void run_to(Stream *s, long number)
-{
-    while (s->done < number) {
-        std::function<void()> f = std::move(s->work.front());
-        s->work.pop_front();
-        f();
-        s->done++;
-    }
-}
 }  // namespace fake
 using fake::error;
 #define LOCK std::lock_guard<std::recursive_mutex> lock(fake::mu)
@@ -56,7 +36,6 @@ using fake::error;
 extern "C" {
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetDeviceFlags(unsigned *f) { *f = 0; return hipSuccess; }
 hipError_t hipGetLastError() { hipError_t e = fake::last; fake::last = hipSuccess; return e; }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 static hipError_t alloc(void **p, size_t n)
@@ -98,39 +77,14 @@ hipError_t hipStreamDestroy(hipStream_t s)
 hipError_t hipStreamSynchronize(hipStream_t s)
 {
     LOCK;
-    fake::Stream *q = fake::streams.at(s);
-    fake::run_to(q, q->queued);
+    std::deque<std::function<void()>> &work = fake::streams.at(s)->work;
+    for (; !work.empty(); work.pop_front()) work.front()();
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st)
 {
     LOCK;
-    fake::push(fake::streams.at(st), [=] { memcpy(d, s, n); });
-    return hipSuccess;
-}
-hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = (hipEvent_t) new fake::Event; return hipSuccess; }
-hipError_t hipEventDestroy(hipEvent_t e) { delete (fake::Event *)e; return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
-{
-    LOCK;
-    fake::Stream *q = fake::streams.at(s);
-    fake::push(q, [] {});
-    ((fake::Event *)e)->on = q;
-    ((fake::Event *)e)->number = q->queued;
-    return hipSuccess;
-}
-hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
-{
-    LOCK;
-    const fake::Event v = *(fake::Event *)e;
-    fake::push(fake::streams.at(s), [v] { fake::run_to(v.on, v.number); });
-    return hipSuccess;
-}
-hipError_t hipEventSynchronize(hipEvent_t e)
-{
-    LOCK;
-    const fake::Event v = *(fake::Event *)e;
-    if (v.on) fake::run_to(v.on, v.number);
+    fake::streams.at(st)->work.push_back([=] { memcpy(d, s, n); });
     return hipSuccess;
 }
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t, hipStream_t s) { fake::calls.push_back({g, b, s}); return hipSuccess; }
@@ -170,7 +124,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **a, size_
     const long c0 = *(long *)a[3];
     const unsigned threads = grid.x * block.x;
     const bool out = f == (const void *)k_piece_to_aos;
-    fake::push(fake::streams.at(st), [=] {
+    fake::streams.at(st)->work.push_back([=] {
         if (out) convert<true>(L, soa, nv, c0, n, aos, threads);
         else convert<false>(L, soa, nv, c0, n, aos, threads);
     });

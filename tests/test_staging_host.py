@@ -43,7 +43,7 @@ def stg(built, tmp_path):
 
 
 MANY = 1 << 40
-SMALL, LARGE = (3, 4, 2), (70, 64, 60)  # one unit, eight units
+SMALL, LARGE = (3, 4, 2), (70, 64, 60)  # one unit, room for eight
 
 
 @pytest.mark.parametrize("shape", [SMALL, (26, 26, 26), (27, 26, 26), (300, 1, 1), LARGE])
@@ -82,3 +82,20 @@ def test_failed_piece_leaves_no_work_behind(stg, shape, launches):
     assert stg.stg_unfinished() == 0
     stg.stg_allow(MANY, MANY)
     assert stg.stg_round_trip(*shape) == 0
+
+
+def test_units_and_streams_are_made_as_transfers_earn_them(stg):
+    """A process that opens one context at a time pays little for units it will hardly use; one that
+    transfers again and again has all of them soon."""
+    assert stg.stg_round_trip(*SMALL) == 0
+    assert (stg.stg_streams_made(), stg.stg_allocs_made()) == (1, 2)  # the context's own stream
+    stg.stg_release()
+    stg.stg_retain()
+    streams, allocs = stg.stg_streams_made(), stg.stg_allocs_made()
+    assert stg.stg_round_trip(*LARGE) == 0
+    assert stg.stg_streams_made() - streams <= 3 and stg.stg_allocs_made() - allocs == 2
+    for _ in range(20):
+        assert stg.stg_round_trip(*LARGE) == 0
+    assert stg.stg_streams_made() - streams == 7 and stg.stg_allocs_made() - allocs == 2
+    stg.stg_release()
+    assert stg.stg_live() == 0
