@@ -1090,6 +1090,9 @@ struct cumc_tape {
     // seg / sa / sb hold the last checkpoint segment, stored by tape_run's own forward pass, so
     // the backward does not re-run that segment (with every >= nsteps it re-runs nothing)
     bool last_stored = false;
+    // the context or batch whose tape_run recorded this tape to its end, null until then: what a
+    // backward pass may reverse
+    const void *by = nullptr;
 };
 static constexpr int SW = 20;  // planes of a stored state
 
@@ -1348,6 +1351,7 @@ extern "C" int cumc_tape_run(cumc_ctx *ctx, int nsteps, int every, const double 
     ctx->dt_valid = false;
     HIPCHK(ctx, hipGetLastError());
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    tp->by = ctx;
     if (dt_out) std::memcpy(dt_out, tp->dts.data(), sizeof(double) * nsteps);
     return CUMC_OK;
 }
@@ -1369,7 +1373,7 @@ extern "C" int cumc_tape_backward(cumc_ctx *ctx, const double *seed_prim, const 
 {
     if (!ctx) return CUMC_EINVAL;
     cumc_tape *tp = ctx->tape;
-    if (!tp) return fail(ctx, CUMC_ESTATE, "cumc_tape_run must precede cumc_tape_backward");
+    if (!tp || tp->by != ctx) return fail(ctx, CUMC_ESTATE, "cumc_tape_run must precede cumc_tape_backward");
     const Lay &L = ctx->L;
     const size_t ps = L.ps, pb = plane_bytes(ctx);
     AdjF &A = tp->A;
@@ -1710,7 +1714,7 @@ __global__ __launch_bounds__(256) void kbr_zfold_bc(Lay L, double *BC)
 }  // namespace
 
 struct batch_tape {
-    bool valid = false;  // a tape is recorded (the allocations and streams below outlive a failed tape_run)
+    bool valid = false;  // a tape is recorded to its end (the allocations and streams below outlive a failed tape_run)
     int nsteps = 0, every = 1, nck = 0, recon = 4;
     std::vector<AdjBox> h;
     AdjBox *d = nullptr;
@@ -1941,7 +1945,11 @@ extern "C" int cumc_batch_tape_run(cumc_batch *b, int nsteps, int every, const d
                 return CUMC_ENONFINITE;
             }
     for (int i = 0; i < nb; i++) BTCHK(b, hipStreamSynchronize(batch_box(b, i)->stream));
-    if (batch_adj(b)) batch_adj(b)->valid = false;
+    if (batch_tape *last = batch_adj(b)) {
+        last->valid = false;
+        last->held[0] = last->held[1] = -1;
+        last->dts.clear();
+    }
     // two sets of segment buffers when the backward re-runs segments (it re-runs one segment
     // while it reverses the next)
     const int sets = nsteps > every ? 2 : 1;
@@ -1956,7 +1964,6 @@ extern "C" int cumc_batch_tape_run(cumc_batch *b, int nsteps, int every, const d
     // the number of boxes)
     if (!batch_adj(b)) batch_adj(b) = new batch_tape();
     batch_tape *bt = batch_adj(b);
-    bt->valid = true;
     bt->recompute_ms = 0.0;
     bt->nsteps = nsteps;
     bt->every = every;
@@ -2031,6 +2038,8 @@ extern "C" int cumc_batch_tape_run(cumc_batch *b, int nsteps, int every, const d
                 batch_err(b) = "box " + std::to_string(i % nb) + ": finddt produced a non-finite step";
                 return CUMC_ENONFINITE;
             }
+    bt->valid = true;
+    for (int i = 0; i < nb; i++) batch_box(b, i)->tape->by = b;
     return CUMC_OK;
 }
 
@@ -2038,11 +2047,14 @@ extern "C" int cumc_batch_tape_backward(cumc_batch *b, const double *const *seed
 {
     if (!b) return CUMC_EINVAL;
     batch_tape *bt = batch_adj(b);
-    if (!bt || !bt->valid) {
+    const int nb = batch_nbox(b);
+    bool recorded = bt && bt->valid;
+    // (a box taped by itself or in another batch since then holds that tape)
+    for (int i = 0; i < nb && recorded; i++) recorded = batch_box(b, i)->tape && batch_box(b, i)->tape->by == b;
+    if (!recorded) {
         batch_err(b) = "cumc_batch_tape_run must precede cumc_batch_tape_backward";
         return CUMC_ESTATE;
     }
-    const int nb = batch_nbox(b);
     hipStream_t s = batch_stream(b);
     // each box is reversed (and its segments re-run) in the view its tape was recorded in,
     // whatever happened to its live state since (uploads, downloads, the collapse switch)

@@ -226,7 +226,8 @@ int cumc_tape_run(cumc_ctx *ctx, int nsteps, int every, const double *dt_in, dou
  * as cumc_download; NULL = zero).  Outputs: gradients with respect to the uploaded prim / eps
  * (cumc_upload layouts; NULL = not wanted).  Recomputes each `every`-step segment but the last
  * from its checkpoint (every >= nsteps: nothing is recomputed); leaves the context at the taped
- * final state. */
+ * final state.  CUMC_ESTATE unless the context's last tape is one that cumc_tape_run recorded to
+ * its end. */
 int cumc_tape_backward(cumc_ctx *ctx, const double *seed_prim, const double *seed_eps, const double *seed_bcell,
                        double *grad_prim, double *grad_eps);
 int cumc_tape_free(cumc_ctx *ctx);
@@ -237,7 +238,8 @@ int cumc_tape_free(cumc_ctx *ctx);
  * are arrays of nbox host pointers (cumc_download / cumc_upload layouts; an array or an entry may
  * be NULL).  cumc_batch_last_ms afterwards gives the device time of the backward pass.  The
  * batched backward re-runs each checkpoint segment but the last two (whose stage states the
- * taping forward keeps in the two sets of segment buffers that the overlapped re-runs use). */
+ * taping forward keeps in the two sets of segment buffers that the overlapped re-runs use).
+ * CUMC_ESTATE unless every box's last tape is the one this batch recorded to its end. */
 int cumc_batch_tape_run(cumc_batch *b, int nsteps, int every, const double *dt_in, double *dt_out);
 int cumc_batch_tape_backward(cumc_batch *b, const double *const *seed_bcell, double *const *grad_prim);
 int cumc_batch_tape_free(cumc_batch *b);
