@@ -1227,9 +1227,9 @@ static void reverse_step(cumc_ctx *ctx, int i, double dt)
 // adjoint arrays and the three conserved-state adjoints
 static int tape_alloc(cumc_ctx *ctx, int nsteps, int every, bool zcollapse_ok = false, int sets = 1)
 {
-    // the last tape's allocation is kept where it serves (and is not four times too large): a training
-    // loop tapes the same map again and again, and 12 boxes of 64^2 to 192^2 took up to 0.3 s a pass to
-    // free and allocate their 20 GB
+    // the last tape's allocation is kept where it is the size this one needs (never larger, so that tapes
+    // take no more memory than what they hold): a training loop tapes the same map again and again, and 12
+    // boxes of 64^2 to 192^2 took up to 0.3 s a pass to free and allocate their 20 GB
     double *mem = nullptr;
     size_t mem_words = 0;
     if (ctx->tape) {
@@ -1253,17 +1253,16 @@ static int tape_alloc(cumc_ctx *ctx, int nsteps, int every, bool zcollapse_ok = 
     const size_t seg_states = sets > 1 ? (size_t)3 * (every + 1) * sets : (size_t)3 * every + 1;
     const size_t planes = 9 + (size_t)SW * tp->nck + (size_t)SW * seg_states + NADJ + 24;
     const size_t words = planes * ps;
-    if (mem_words < words || mem_words / 4 > words) {
+    if (mem_words != words) {
         hipFree(mem);
         mem = nullptr;
-        mem_words = words;
         if (hipMalloc(&mem, words * sizeof(double)) != hipSuccess) {
             tape_release(ctx);
             return fail(ctx, CUMC_ENOMEM, "tape allocation");
         }
     }
     tp->mem = mem;
-    tp->mem_words = mem_words;
+    tp->mem_words = words;
     double *p = tp->mem;
     auto take = [&](size_t n) { double *r = p; p += n * ps; return r; };
     tp->init = take(9);

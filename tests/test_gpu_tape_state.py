@@ -76,3 +76,58 @@ def test_a_box_holds_one_tape():
     solvers[0].tape_free()
     _refused(lambda: b.tape_backward(seeds))
     _refused(lambda: solvers[0].tape_backward(seed_bcell=seeds[0]))
+
+
+# (steps, checkpoint interval): again the same, fewer in what the last one held, more, one set of segment
+# buffers after two, none re-run after some
+TAPES = [(8, 4), (8, 4), (3, 4), (12, 2), (12, 2), (1, 1), (8, 4), (2, 8)]
+
+
+def _fresh_gradients(probs, seeds, steps, every):
+    from cumpic_amd.cumc import Batch, Solver
+    solvers = [Solver.from_problem(p) for p in probs]
+    b = Batch(solvers)
+    b.tape_run(steps, every)
+    return b.tape_backward(seeds)
+
+
+def test_gradients_do_not_depend_on_earlier_tapes():
+    """Memory kept from one tape to the next: every gradient is a fresh object's bit for bit, for one box and
+    for a batch, and for a box used alone between two batch tapes."""
+    from cumpic_amd.cumc import Batch, Solver
+    probs = [_box(16, 6), _box(24, 7)]
+    seeds = _seeds(probs)
+    solvers = [Solver.from_problem(p) for p in probs]
+    b = Batch(solvers)
+    for steps, every in TAPES:
+        want = _fresh_gradients(probs, seeds, steps, every)
+        one = Solver.from_problem(probs[1])
+        one.tape_run(steps, every)
+        alone = one.tape_backward(seed_bcell=seeds[1])[0]
+        for s, p in zip(solvers, probs):
+            s.upload(p.prim, p.eps)
+        b.tape_run(steps, every)
+        for i, g in enumerate(b.tape_backward(seeds)):
+            assert np.array_equal(g, want[i]), f"batch, {steps} steps every {every}, box {i}"
+        solvers[1].upload(probs[1].prim, probs[1].eps)
+        solvers[1].tape_run(steps, every)
+        assert np.array_equal(solvers[1].tape_backward(seed_bcell=seeds[1])[0], alone), f"alone, {steps} every {every}"
+
+
+def _free_bytes():
+    import ctypes
+    from cumpic_amd.cumc import lib
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_a_small_tape_gives_a_large_one_back():
+    """A tape holds what it needs: device memory after a small tape does not depend on one before it."""
+    from cumpic_amd.cumc import Solver
+    s = Solver.from_problem(_box(256, 8))
+    s.tape_run(1, 1)
+    free = _free_bytes()
+    s.tape_run(4, 4)  # about 1.7 times the states
+    s.tape_run(1, 1)
+    assert _free_bytes() >= free - (8 << 20)
