@@ -257,7 +257,7 @@ def timed_run(Solver, prob, prec, steps, warmup, tune=True):
     if warmup:
         s.run(warmup)
     tuning = s.autotune() if tune else s.tuning()
-    s.profile(True)
+    s.profile(True, joined=True)
     t0 = time.perf_counter()
     dts, _ = s.run(steps)  # synchronous on return (hipStreamSynchronize)
     wall = time.perf_counter() - t0
@@ -267,7 +267,7 @@ def timed_run(Solver, prob, prec, steps, warmup, tune=True):
 
 
 def roofline(kt, cfg, tag, traffic=None):
-    """Roofline of the stage tail, the kernel that takes the most time: algorithmic bytes per
+    """Roofline of the stage tail, the kernel that takes the most HBM time: algorithmic bytes per
     launch = 512/3 B per interior zone (one stage's share of the RK3 state traffic) over its
     average HIP-event launch time, against 8 TB/s.  `traffic` is the HBM bytes per launch that
     the counters of this run measured (None: not measured); kernel_io gives the same launch
@@ -831,7 +831,7 @@ def main():
              "roofline": roofline(kt, cfg, form, traffic=tr),
              "step_traffic_bytes_per_zone_cycle": (tr["step_bytes"] / cfg.zones) if tr else None,
              "traffic_bytes_per_launch_by_kernel": tr["bytes_per_launch_by_class"] if tr else None,
-             "kernel_ms_per_step": {k: v[0] / steps for k, v in kt.items()}, "divb_max_abs": dabs,
+             "kernel_ms_per_step": {k: v[0] / steps for k, v in kt.items() if v[1]}, "divb_max_abs": dabs,
              "state_finite": finite, "tuning": tuning}
         kio = r["roofline"]["kernel_io"]
         if copy_gbps:

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -50,8 +51,9 @@ struct cumc_ctx {
     int tile_w = 0;   // column tile width of those kernels (0: flattened rows; see col_of)
     double last_ms = 0.0;
     std::string err;
-    // per-kernel-class HIP event timing (cumc_profile / cumc_kernel_times)
-    bool prof = false;
+    // per-kernel-class HIP event timing (cumc_profile / cumc_kernel_times): 0 off, 1 with the three FP64
+    // sweeps launched one by one, 2 with the launches of a run
+    int prof = 0;
     std::vector<hipEvent_t> evpool;
     std::vector<int> evcls;
     size_t evn = 0;
@@ -59,8 +61,8 @@ struct cumc_ctx {
     long kc_count[16] = {0};
 };
 
-enum { KC_FLUX_X, KC_FLUX_Y, KC_FLUX_Z, KC_ECORN, KC_TAIL, KC_GHOST, KC_FINDDT, KC_N };
-static const char *kc_names[KC_N] = {"flux_x", "flux_y", "flux_z", "ecorn", "tail", "ghost", "finddt"};
+enum { KC_FLUX_X, KC_FLUX_Y, KC_FLUX_Z, KC_ECORN, KC_TAIL, KC_GHOST, KC_FINDDT, KC_FLUX_XYZ, KC_N };
+static const char *kc_names[KC_N] = {"flux_x", "flux_y", "flux_z", "ecorn", "tail", "ghost", "finddt", "flux_xyz"};
 
 // record the start (cls >= 0) or end (cls < 0) of a kernel class on the context stream
 static inline void mark(cumc_ctx *ctx, int cls)
@@ -183,8 +185,8 @@ void launch_ghost32(cumc_ctx *ctx, int st);
 // (the fourth shares a SIMD), 1.4 to 2.4 from four to eleven, 0.21 m from twelve on; a unit holds 12
 // wavefronts at a time (FP32 20), and more run in rounds of that size.  The plan takes the segment
 // length of least estimated time, at most the tuned one (cumc_tuning.seg), for sweeps launched one by
-// one (the mixed form, profiling).  Per y / z launch, 24-face
-// segments against the plan's: 48^3 46 -> 15.4 us, 96^3 86 -> 49, 128^3 132 / 108 -> 93 / 92,
+// one (the mixed form, one sweep's fluxes, sweeps timed by themselves).  Per y / z launch, 24-face segments
+// against the plan's: 48^3 46 -> 15.4 us, 96^3 86 -> 49, 128^3 132 / 108 -> 93 / 92,
 // torus 128x64x128 80 / 92 -> 50 / 53; 256^3 keeps 24.
 // ------------------------------------------------------------------------------------------
 struct WalkSet {
@@ -237,6 +239,20 @@ static inline int one_launch_seg(long face_waves, int tuned)
     return (int)(s < tuned ? s : tuned);
 }
 
+// The mixed form's y sweep with few pencils: the wave-parallel one, below a fixed line in segments of the
+// tuned length (the two FP32 forms contract different products, so the choice shows in the last bit).
+static inline bool y_lanes(const Lay &L, int seg)
+{
+    return L.ny >= 16 && (long)L.px * flux_planes(L) * nblk(L.ny + 1, seg) < YLANE_WALKERS;
+}
+// What the tuned segment length comes to in the y and z sweeps of a run: values that come to the same are one
+// launch shape, which the tuner times once.
+static inline std::array<int, 3> seg_shape(const Lay &L, bool mixed, int seg)
+{
+    if (!mixed) return {one_launch_seg(sweep_face_waves(L), seg), 0, 0};
+    return {y_lanes(L, seg) ? 0 : walk_plan<float>(walk_set<float>(L, 2), seg), walk_plan<float>(walk_set<float>(L, 3), seg), 0};
+}
+
 template <typename R, int RECON, int SOLVER>
 void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_dir)
 {
@@ -245,8 +261,7 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
     const Model &M = ctx->M;
     const int npl = flux_planes(L);
     if constexpr (sizeof(R) == 8) {
-        // (profiling times the three sweeps one by one)
-        if (!only_dir && !ctx->prof) {
+        if (!only_dir && ctx->prof != 1) {
             const long xw = x_waves(L);
             const WalkSet wy = walk_set<R>(L, 2), wz = walk_set<R>(L, 3);
             SweepGrid G;
@@ -259,8 +274,10 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
             G.z_sl = L.zc1 ? 1 : (wz.faces + nz - 1) / nz;
             G.z_n = G.z_gx * nz;
             G.x_waves = (int)xw;
+            mark(ctx, KC_FLUX_XYZ);
             hipLaunchKernelGGL((k_flux_xyz<RECON, SOLVER>), dim3((unsigned)(G.y_n + G.z_n + xw * npl)), dim3(64), 0, s, L, F,
                                tb, M, G);
+            mark(ctx, -1);
             return;
         }
     }
@@ -274,12 +291,7 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
     if (!only_dir || only_dir == 2) {
         mark(ctx, KC_FLUX_Y);
         const int psl = walk_plan<R>(walk_set<R>(L, 2), seg);
-        bool lanes = false;
-        if constexpr (sizeof(R) == 4) {
-            // few pencils: the wave-parallel y sweep, below a fixed line in segments of the tuned length
-            // (the two FP32 forms contract different products, so the choice shows in the last bit)
-            lanes = L.ny >= 16 && (long)L.px * npl * nblk(L.ny + 1, seg) < YLANE_WALKERS;
-        }
+        const bool lanes = sizeof(R) == 4 && y_lanes(L, seg);
         if (lanes) {
             if constexpr (sizeof(R) == 4) {
                 const int gx = ylane_groups(L) * ylane_segs(L);

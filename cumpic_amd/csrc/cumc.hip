@@ -4,6 +4,7 @@
 // buffer; host arrays crossing the ABI are caller-owned and in the reference's Fortran layout.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -791,11 +792,12 @@ extern "C" int cumc_set_tuning(cumc_ctx *ctx, const cumc_tuning *t)
     return CUMC_OK;
 }
 
-// Tuner: one warm-up step, then one timed step per candidate with per-kernel-class HIP events:
-// the segment length is scored by the y + z sweeps, the plane chunk and column tiles by the EMF +
-// stage-tail kernels.  The FP64 fields (and the mixed form's FP32 primitive planes), the dt slots and the
-// U0/U1 assignment are saved and restored, so the state is as before; the per-class timing
-// totals are cleared.
+// Tuner: one warm-up step, then one timed step per launch shape with per-kernel-class HIP events, in the
+// launches of a run: the segment length is scored by the sweeps, the plane chunk and column tiles by the EMF +
+// stage-tail kernels.  Candidates that come to a launch shape timed before (the sweeps, the tail and the EMF
+// kernel cap what they take) are left out, and the present values are first, so that where all are one shape
+// they stay.  The FP64 fields (and the mixed form's FP32 primitive planes), the dt slots and the U0/U1
+// assignment are saved and restored, so the state is as before; the per-class timing totals are cleared.
 extern "C" int cumc_autotune(cumc_ctx *ctx, cumc_tuning *out)
 {
     if (!ctx) return CUMC_EINVAL;
@@ -806,7 +808,8 @@ extern "C" int cumc_autotune(cumc_ctx *ctx, cumc_tuning *out)
     if (hipMalloc(&save, ctx->pool_bytes + p32_bytes) != hipSuccess) return fail(ctx, CUMC_ENOMEM, "tuner state copy");
     double dts[2];
     double *u0 = ctx->F64.U0, *u1 = ctx->F64.U1;
-    const bool valid = ctx->dt_valid, prof = ctx->prof, stale = ctx->p64_stale;
+    const bool valid = ctx->dt_valid, stale = ctx->p64_stale;
+    const int prof = ctx->prof;
     const bool zmode0 = ctx->zmode, zfresh0 = ctx->zfresh;
     const int seg0 = ctx->seg, zc0 = ctx->zchunk, tw0 = ctx->tile_w;
     hipMemcpyAsync(save, ctx->pool, ctx->pool_bytes, hipMemcpyDeviceToDevice, ctx->stream);
@@ -818,7 +821,7 @@ extern "C" int cumc_autotune(cumc_ctx *ctx, cumc_tuning *out)
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) rc = fail(ctx, CUMC_EHIP, "tuner state copy");
     if (rc == CUMC_OK) rc = finddt_to_current(ctx, &dt);
     auto timed_step = [&](double *cls) -> int {
-        ctx->prof = true;
+        ctx->prof = 2;
         ctx->evn = 0;
         for (int c = 0; c < KC_N; c++) ctx->kc_ms[c] = 0.0;
         hipMemcpyAsync(ctx->dt_dev, &dt, sizeof(double), hipMemcpyHostToDevice, ctx->stream);
@@ -831,37 +834,34 @@ extern "C" int cumc_autotune(cumc_ctx *ctx, cumc_tuning *out)
     double cls[KC_N];
     int best_seg = seg0, best_zc = zc0, best_tw = tw0;
     if (rc == CUMC_OK) rc = timed_step(cls);  // warm-up
-    if (rc == CUMC_OK) {
-        const int segs[] = {8, 12, 16, 24, 32, 48, 64, 96};
+    // the candidate of least time of the given classes, each shape once, the present value first
+    auto pick = [&](int &knob, std::initializer_list<int> cands, auto shape, std::initializer_list<int> classes) {
+        const int now = knob;
+        int best = now;
         double bt = 1e300;
-        for (int sg : segs) {
-            ctx->seg = sg;
-            if ((rc = timed_step(cls))) break;
-            const double v = cls[KC_FLUX_Y] + cls[KC_FLUX_Z];
-            if (v < bt) { bt = v; best_seg = sg; }
-        }
-        ctx->seg = best_seg;
-    }
+        std::vector<decltype(shape(now))> seen;
+        auto time = [&](int v) {
+            if (rc != CUMC_OK || std::find(seen.begin(), seen.end(), shape(v)) != seen.end()) return;
+            seen.push_back(shape(v));
+            knob = v;
+            if ((rc = timed_step(cls))) return;
+            double t = 0.0;
+            for (int c : classes) t += cls[c];
+            if (t < bt) { bt = t; best = v; }
+        };
+        time(now);
+        for (int v : cands) time(v);
+        knob = best;
+        return best;
+    };
     if (rc == CUMC_OK) {
-        const int zcs[] = {1, 2, 4, 8, 16, 32};
-        double bt = 1e300;
-        for (int z : zcs) {
-            ctx->zchunk = z;
-            if ((rc = timed_step(cls))) break;
-            const double v = cls[KC_ECORN] + cls[KC_TAIL];
-            if (v < bt) { bt = v; best_zc = z; }
-        }
-        ctx->zchunk = best_zc;
-    }
-    if (rc == CUMC_OK) {
-        const int tws[] = {0, 32, 64, 128};
-        double bt = 1e300;
-        for (int w : tws) {
-            ctx->tile_w = w;
-            if ((rc = timed_step(cls))) break;
-            const double v = cls[KC_ECORN] + cls[KC_TAIL];
-            if (v < bt) { bt = v; best_tw = w; }
-        }
+        const Lay L = make_view(ctx, ctx->zmode).L;
+        const bool mixed = ctx->cfg.precision == CUMC_MIXED;
+        best_seg = pick(ctx->seg, {8, 12, 16, 24, 32, 48, 64, 96}, [&](int v) { return seg_shape(L, mixed, v); },
+                        {KC_FLUX_XYZ, KC_FLUX_Y, KC_FLUX_Z});
+        best_zc = pick(ctx->zchunk, {1, 2, 3}, [&](int v) {
+            return std::array<int, 2>{tail_chunk(L, v, ctx->tile_w), ecorn_chunk(L, v, ctx->tile_w)}; }, {KC_ECORN, KC_TAIL});
+        best_tw = pick(ctx->tile_w, {0, 32, 64, 128}, [](int v) { return v; }, {KC_ECORN, KC_TAIL});
     }
     hipMemcpyAsync(ctx->pool, save, ctx->pool_bytes, hipMemcpyDeviceToDevice, ctx->stream);
     if (p32_bytes)
@@ -926,7 +926,7 @@ extern "C" int cumc_profile(cumc_ctx *ctx, int on)
         ctx->kc_ms[c] = 0.0;
         ctx->kc_count[c] = 0;
     }
-    ctx->prof = on != 0;
+    ctx->prof = on == 2 ? 2 : on != 0;
     return CUMC_OK;
 }
 
@@ -954,7 +954,7 @@ __global__ __launch_bounds__(256) void k_copy_probe(const double2 *__restrict__ 
 }
 
 // The stage tail's memory access pattern with no arithmetic: NR FP64 planes read and NW written
-// at each cell, one (j,k) column per thread over a chunk of planes, with the tail's column tiles
+// at each cell, one (j,k) column per thread over the tail's chunk of planes (tail_chunk), with its column tiles
 // and XCD tile order.  Its bandwidth is the ceiling the tail itself can reach on this layout.
 template <int NR, int NW>
 __global__ __launch_bounds__(256) void k_pattern_probe(Lay L, const double *__restrict__ in, double *__restrict__ out,
@@ -983,8 +983,8 @@ extern "C" int cumc_pattern_probe(cumc_ctx *ctx, int nread, int nwrite, int reps
 {
     if (!ctx || reps < 1 || !gbps) return CUMC_EINVAL;
     const Lay &L = ctx->L;
-    const int zc = ctx->zchunk, tw = ctx->tile_w;
-    const int gx = col_tiles(L, tw), gy = (L.nz + zc) / zc;
+    const int tw = ctx->tile_w, zc = tail_chunk(L, ctx->zchunk, tw);
+    const int gx = col_tiles(L, tw), gy = zchunks(L, zc);
     const dim3 grid(xcd_blocks(gx, gy));
     void (*kern)(Lay, const double *, double *, int, int, int, int) = nullptr;
     if (nread == 26 && nwrite == 20) kern = k_pattern_probe<26, 20>;

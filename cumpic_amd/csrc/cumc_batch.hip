@@ -14,6 +14,7 @@
 // multi-step run can be replayed from one graph.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -741,11 +742,19 @@ extern "C" int cumc_batch_autotune(cumc_batch *b, cumc_tuning *out)
     }
     cumc_tuning best = orig;
     if (rc == CUMC_OK && hipStreamSynchronize(b->stream) != hipSuccess) rc = bfail(b, CUMC_EHIP, "tuner sync");
+    if (rc == CUMC_OK) rc = refresh(b);
     // 1) segment length of the pencil sweeps (one workgroup per tile)
     if (rc == CUMC_OK) {
-        const int segs[] = {8, 12, 16, 24, 32, 64, 128, 256};
+        // (candidates that come to a length timed before are the same launch; the present value is first)
+        long face_waves = 0;
+        for (const BoxDesc &d : b->h_desc) face_waves += sweep_face_waves(d.L);
+        const int segs[] = {orig.seg > 0 ? orig.seg : 24, 8, 12, 16, 24, 32, 64, 128, 256};
+        std::vector<int> seen;
         double bestt = 1e300;
         for (int sg : segs) {
+            const int sl = one_launch_seg(face_waves, sg);
+            if (std::find(seen.begin(), seen.end(), sl) != seen.end()) continue;
+            seen.push_back(sl);
             cumc_tuning t = orig;
             t.seg = sg;
             for (int p = 0; p < CUMC_PH_N; p++) t.blocks[p] = 0;
@@ -760,7 +769,7 @@ extern "C" int cumc_batch_autotune(cumc_batch *b, cumc_tuning *out)
     }
     // 2) plane chunk and column tile shape of the EMF / tail kernels
     if (rc == CUMC_OK) {
-        const int zcs[] = {1, 2, 4, 8, 32};
+        const int zcs[] = {1, 2, 3};  // (the tail takes at most 2, the EMF kernel at most 3)
         double bestt = 1e300;
         for (int z : zcs) {
             cumc_tuning t = best;

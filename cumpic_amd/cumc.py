@@ -233,8 +233,9 @@ class Solver:
         self._check(self._L.cumc_sweep_flux(self.h, int(direction), _p(out)), "cumc_sweep_flux")
         return out
 
-    def profile(self, on: bool = True):
-        self._check(self._L.cumc_profile(self.h, 1 if on else 0), "cumc_profile")
+    def profile(self, on: bool = True, joined: bool = False):
+        """HIP-event timing per kernel class: of the FP64 sweeps one by one, or joined, as a run launches them."""
+        self._check(self._L.cumc_profile(self.h, (2 if joined else 1) if on else 0), "cumc_profile")
 
     def kernel_times(self):
         """{class: (total_ms, launches)} of the HIP-event timing since profile(True)."""

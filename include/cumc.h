@@ -115,8 +115,10 @@ int cumc_last_step_ms(cumc_ctx *ctx, double *ms);
 
 /* Per-kernel-class timing with HIP events recorded on the context stream around every launch
  * group (no reference counterpart; the reference has no timers).  cumc_profile(ctx, 1) clears
- * and enables it; cumc_kernel_times fills up to n entries of total milliseconds, launch counts
- * and class names, and returns the number of classes. */
+ * and enables it with the three FP64 sweeps launched and timed one by one (flux_x, flux_y, flux_z);
+ * cumc_profile(ctx, 2) with the launches of a run, the FP64 sweeps in one (flux_xyz).
+ * cumc_kernel_times fills up to n entries of total milliseconds, launch counts and class names,
+ * and returns the number of classes. */
 int cumc_profile(cumc_ctx *ctx, int on);
 int cumc_kernel_times(cumc_ctx *ctx, int n, double *total_ms, long *launches, const char **names);
 
@@ -126,7 +128,7 @@ int cumc_kernel_times(cumc_ctx *ctx, int n, double *total_ms, long *launches, co
 int cumc_copy_probe(long bytes, int reps, double *gbps);
 
 /* Diagnostic, no reference counterpart: the stage tail's memory access pattern on this context's
- * layout and tuned column tiles, with no arithmetic -- `nread` FP64 planes read and `nwrite`
+ * layout, column tiles and plane chunks, with no arithmetic -- `nread` FP64 planes read and `nwrite`
  * written per cell of [0,n]^3, run `reps` times; reports (nread + nwrite) * 8 bytes per cell per
  * second in GB/s, the bandwidth ceiling of a kernel with that access pattern.  Supported
  * (nread, nwrite): (26, 20) and (34, 20) (the FP64 tail of stage 1 and of stages 2-3), (34, 0)
@@ -143,15 +145,18 @@ const char *cumc_last_error(cumc_ctx *ctx);
 enum { CUMC_PH_FLUX_X = 0, CUMC_PH_FLUX_Y, CUMC_PH_FLUX_Z, CUMC_PH_ECORN, CUMC_PH_TAIL, CUMC_PH_GHOST,
        CUMC_PH_FINDDT, CUMC_PH_N };
 typedef struct cumc_tuning {
-    int seg;                 /* most faces per pencil segment of the y and z sweeps */
-    int zchunk;              /* most planes per column tile of the EMF and stage-tail kernels */
+    int seg;                 /* most faces per pencil segment of the y and z sweeps: small grids take
+                                shorter ones whatever this is */
+    int zchunk;              /* most planes per column tile of the EMF kernel (which takes up to 3) and the
+                                stage tail (up to 2); small grids take 1 */
     int blocks[CUMC_PH_N];   /* batch only: persistent workgroups per phase, 0 = one per tile */
     int tile_w;              /* column tile of the EMF / stage-tail kernels: 0 = flattened rows of 256
                                 cells, or 32 / 64 / 128 = tile_w x (256 / tile_w) columns */
 } cumc_tuning;
 
-/* Time candidate shapes on the context's current state (which is saved and restored) and keep
- * the fastest; *out (may be NULL) receives the choice. */
+/* Time candidate shapes, in the launches of a run, on the context's current state (which is saved and
+ * restored) and keep the fastest; *out (may be NULL) receives the choice.  A value whose candidates all
+ * come to the same launches is left as it is. */
 int cumc_autotune(cumc_ctx *ctx, cumc_tuning *out);
 int cumc_get_tuning(cumc_ctx *ctx, cumc_tuning *out);
 int cumc_set_tuning(cumc_ctx *ctx, const cumc_tuning *t);

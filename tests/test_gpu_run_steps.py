@@ -64,3 +64,32 @@ def test_run_stops_at_a_non_finite_step():
     s.initial_update()
     fresh = _start("box", FP64)
     assert_bitwise(s.run(9)[0], fresh.run(9)[0], "dt after the error")
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_profile_counts_the_launches_it_says(mixed):
+    from cumpic_amd.config import FP64, MIXED
+    from cumpic_amd.cumc import Solver
+    s = Solver.from_problem(ics.spectral_box(n=20, seed=3), precision=MIXED if mixed else FP64)
+    s.initial_update()
+    sweeps = ("flux_x", "flux_y", "flux_z", "flux_xyz")
+    for joined in (False, True):
+        s.profile(True, joined=joined)
+        s.run(2)
+        n = {k: v[1] for k, v in s.kernel_times().items()}
+        assert [n[k] for k in sweeps] == ([0, 0, 0, 6] if joined and not mixed else [6, 6, 6, 0])
+        assert n["tail"] == n["ecorn"] == n["ghost"] == 6
+
+
+def test_tuner_leaves_values_that_change_no_launch():
+    """On a small grid every segment length and plane chunk comes to one face and one plane: nothing to choose."""
+    from cumpic_amd.cumc import Batch, Solver
+    solvers = [Solver.from_problem(ics.small_periodic(8)) for _ in range(2)]
+    for s in solvers:
+        s.initial_update()
+    solvers[0].set_tuning({**solvers[0].tuning(), "seg": 17, "zchunk": 5})
+    t = solvers[0].autotune()
+    assert (t["seg"], t["zchunk"]) == (17, 5)
+    b = Batch(solvers)
+    seg = b.tuning()["seg"]
+    assert b.autotune()["seg"] == (seg if seg > 0 else 24)
