@@ -140,6 +140,7 @@ static inline void swap_u(cumc_ctx *ctx)
 struct DtHandOn {
     cumc_ctx *ctx;
     bool pending = false;  // a step that will publish is enqueued
+    bool block = false;    // the device is set to blocking waits (hipDeviceScheduleBlockingSync)
     DtHandOn(cumc_ctx *c, bool on);
     ~DtHandOn() { ctx->dt_pub = nullptr; }
     int next(double *dt);  // dt of the current state, in dt_dev[0] too

@@ -1,4 +1,8 @@
 """Steps of one run, which hand the time step on by themselves, against steps called one by one."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -7,6 +11,8 @@ from cumpic_amd.config import FP64, MIXED
 from tests.helpers import assert_bitwise
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..")
 
 PROBLEMS = {
     "box": lambda: ics.randomize(ics.small_periodic(17, seed=5), seed=6, amp=0.1),
@@ -93,3 +99,25 @@ def test_tuner_leaves_values_that_change_no_launch():
     b = Batch(solvers)
     seg = b.tuning()["seg"]
     assert b.autotune()["seg"] == (seg if seg > 0 else 24)
+
+
+BLOCKING = """
+import time
+from cumpic_amd import ics
+from cumpic_amd.cumc import Solver, lib
+assert lib().hipSetDeviceFlags(4) == 0  # hipDeviceScheduleBlockingSync
+s = Solver.from_problem(ics.spectral_box(n=128))
+s.initial_update()
+s.run(20)
+wall, cpu = time.perf_counter(), time.process_time()
+s.run(100)
+print(time.process_time() - cpu, time.perf_counter() - wall)
+"""
+
+
+def test_run_waits_as_the_device_is_set_to():
+    """With blocking waits chosen, a run's steps leave the core to others (watching takes all of it)."""
+    out = subprocess.run([sys.executable, "-c", BLOCKING], cwd=ROOT, stdout=subprocess.PIPE, text=True, timeout=100)
+    assert out.returncode == 0
+    cpu, wall = (float(v) for v in out.stdout.split())
+    assert cpu < 0.75 * wall
