@@ -508,10 +508,140 @@ __device__ inline void flux_walk_tile(const Lay &L, const Fields<R> &F, const Ta
     }
 }
 
+// The FP32 walk of WENO5, of HLLD and of HLLC behind TVD: each cell loaded as it is needed, both face values
+// of a cell formed in it, and the face's products contracted as the compiler sees fit.  Sharing face values and
+// loading ahead moved the compiler's choice of which product to round (the mixed form may contract), and the
+// products that vsq_side to sub_sq name are HLL's, LF's and PPM + HLLC's: there every flux is what this walk
+// gives, bit for bit, while WENO5's z fluxes were 1.5 to 2 % further from the FP64 ones (rel L1 3.97e-7 against
+// 3.90e-7 with this walk) and HLLD took other branches.  Loading ahead was worth nothing there from 96^3 up
+// (WENO5 + HLL 741 us a step against 736) and 2 % at 24^3 and 48^3.
+template <int RECON, int SOLVER>
+constexpr bool plain_walk() { return RECON == 5 || SOLVER == 4 || (SOLVER == 3 && RECON != 4); }
+template <int DIR, int RECON, int SOLVER>
+__device__ inline void flux_walk_plain(const Lay &L, const Fields<float> &F, const Tabs &tb, const Model &M, int seglen,
+                                       int bx, int by)
+{
+    using R = float;
+    const long t = (long)bx * blockDim.x + threadIdx.x;
+    const int nd = DIR == 2 ? L.ny : L.nz, nt = DIR == 2 ? L.nz : L.ny;
+    const int jj = (int)(t % L.px);
+    const long tq = t / L.px;
+    const int j = jj - 2;
+    if (tq > nt + 1 || j < 0 || j > L.nx + 1) return;
+    const int s0 = by * seglen;
+    if (s0 > nd) return;
+    const int s1 = (s0 + seglen - 1 < nd) ? s0 + seglen - 1 : nd;
+    const unsigned stride = (unsigned)(DIR == 2 ? L.px : L.py);
+    const unsigned base = (unsigned)(DIR == 2 ? (long)(tq + 2) * L.py + 2 + j : (long)(tq + 2) * L.px + 2 + j);
+    auto at = [&](int c) { return base + (unsigned)(c + 2) * stride; };
+    const long ps = L.ps;
+    const int ax = DIR - 1, bB = DIR == 2 ? 2 : 1, ibn = DIR == 2 ? 6 : 7;
+    auto load7 = [&](int c, R *o) {
+        const unsigned g = at(c);
+        const R *SP = sweep_p(F), *SB = sweep_bc(F);
+        o[0] = ldi(SP, g);
+        o[1] = ldi(SP + ps, g);
+        o[2] = ldi(SP + 2 * ps, g);
+        o[3] = ldi(SP + 3 * ps, g);
+        o[4] = ldi(SP + 4 * ps, g);
+        o[5] = ldi(SB, g);
+        o[6] = ldi(SB + bB * ps, g);
+    };
+    // window: w0 = v(c-1), w1 = v(c), w2 = v(c+1), w3 = v(c+2), wm = v(c-2); PPM: d0, d1, d2 = slopes of c-1, c, c+1
+    R w0[7], w1[7], w2[7], w3[7], d0[7], d1[7], vpp[7];
+    R wm[RECON == 5 ? 7 : 1];
+    {
+        R a[7];
+        load7(s0 - 2, a);
+        load7(s0 - 1, w0);
+        load7(s0, w1);
+        load7(s0 + 1, w2);
+        if (RECON == 5) {
+#pragma unroll
+            for (int v = 0; v < 7; v++) wm[v] = a[v];
+        }
+        if (RECON == 4) {
+            R b0 = tb.atr<R>(ax, TB_B0C, s0 - 1), b1 = tb.atr<R>(ax, TB_B1C, s0 - 1);
+            R c0 = tb.atr<R>(ax, TB_B0C, s0), c1 = tb.atr<R>(ax, TB_B1C, s0);
+#pragma unroll
+            for (int v = 0; v < 7; v++) {
+                d0[v] = ppm_slope<R>(b0, b1, a[v], w0[v], w1[v]);
+                d1[v] = ppm_slope<R>(c0, c1, w0[v], w1[v], w2[v]);
+            }
+        }
+    }
+    for (int c = s0; c <= s1 + 1; c++) {
+        load7(c + 2, w3);
+        R vm[7], vp[7];
+        if (RECON == 5) {
+#pragma unroll
+            for (int v = 0; v < 7; v++) weno5_edges<R>(wm[v], w0[v], w1[v], w2[v], w3[v], vm[v], vp[v]);
+            weno_positivity<R>(w1, vm, vp);
+        } else if (RECON == 4) {
+            R b0 = tb.atr<R>(ax, TB_B0C, c + 1), b1 = tb.atr<R>(ax, TB_B1C, c + 1);
+            R a0m = tb.atr<R>(ax, TB_A0M, c), a1m = tb.atr<R>(ax, TB_A1M, c), a2m = tb.atr<R>(ax, TB_A2M, c);
+            R a3m = tb.atr<R>(ax, TB_A3M, c), a0p = tb.atr<R>(ax, TB_A0P, c), a1p = tb.atr<R>(ax, TB_A1P, c);
+            R a2p = tb.atr<R>(ax, TB_A2P, c), a3p = tb.atr<R>(ax, TB_A3P, c);
+#pragma unroll
+            for (int v = 0; v < 7; v++) {
+                R d2 = ppm_slope<R>(b0, b1, w1[v], w2[v], w3[v]);
+                ppm_edges<R>(a0m, a1m, a2m, a3m, a0p, a1p, a2p, a3p, w0[v], w1[v], w2[v], d0[v], d1[v], d2, vm[v], vp[v]);
+                d0[v] = d1[v];
+                d1[v] = d2;
+            }
+        } else {
+            R cf = tb.atr<R>(ax, TB_CF, c), cb = tb.atr<R>(ax, TB_CB, c);
+#pragma unroll
+            for (int v = 0; v < 7; v++) tvd_any<R, RECON>(cf, cb, w0[v], w1[v], w2[v], vm[v], vp[v]);
+        }
+        if (c > s0) {
+            const unsigned gf = at(c - 1);
+            const R bn = ldi(sweep_p(F) + ibn * ps, gf);
+            R fl[7];
+            if (DIR == 2) {
+                FaceState<R> sl{vpp[0], vpp[2], vpp[3], vpp[1], vpp[4], bn, vpp[6], vpp[5]};
+                FaceState<R> sr{vm[0], vm[2], vm[3], vm[1], vm[4], bn, vm[6], vm[5]};
+                riemann_face<2, R, SOLVER>(R(M.ggas), sl, sr, fl);
+                R *o = F.F[1];
+                sti(o, gf, fl[0]);
+                sti(o + 1 * ps, gf, fl[3]);
+                sti(o + 2 * ps, gf, fl[1]);
+                sti(o + 3 * ps, gf, fl[2]);
+                sti(o + 4 * ps, gf, fl[4]);
+                sti(o + 5 * ps, gf, fl[6]);
+                sti(o + 6 * ps, gf, fl[5]);
+            } else {
+                FaceState<R> sl{vpp[0], vpp[3], vpp[1], vpp[2], vpp[4], bn, vpp[5], vpp[6]};
+                FaceState<R> sr{vm[0], vm[3], vm[1], vm[2], vm[4], bn, vm[5], vm[6]};
+                riemann_face<3, R, SOLVER>(R(M.ggas), sl, sr, fl);
+                R *o = F.F[2];
+                sti(o, gf, fl[0]);
+                sti(o + 1 * ps, gf, fl[2]);
+                sti(o + 2 * ps, gf, fl[3]);
+                sti(o + 3 * ps, gf, fl[1]);
+                sti(o + 4 * ps, gf, fl[4]);
+                sti(o + 5 * ps, gf, fl[5]);
+                sti(o + 6 * ps, gf, fl[6]);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 7; v++) {
+            if (RECON == 5) wm[v] = w0[v];
+            vpp[v] = vp[v];
+            w0[v] = w1[v];
+            w1[v] = w2[v];
+            w2[v] = w3[v];
+        }
+    }
+}
+
 template <typename R, int DIR, int RECON, int SOLVER>
 __global__ __launch_bounds__(walk_block<R>(), (sizeof(R) == 8 ? sweep_waves<RECON, SOLVER>() : 1)) void k_flux_walk(Lay L, Fields<R> F, Tabs tb, Model M, int seglen)
 {
-    flux_walk_tile<R, DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
+    if constexpr (sizeof(R) == 4 && plain_walk<RECON, SOLVER>())
+        flux_walk_plain<DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
+    else
+        flux_walk_tile<R, DIR, RECON, SOLVER>(L, F, tb, M, seglen, blockIdx.x, blockIdx.y);
 }
 
 // The three FP64 sweeps in one launch: they read the same state and write their own planes, by itself

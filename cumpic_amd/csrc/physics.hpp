@@ -383,10 +383,13 @@ __host__ __device__ inline R dot_xyz(R an, R at1, R at2, R bn, R bt1, R bt2)
     else return at1 * bt1 + at2 * bt2 + an * bn;                 // (x,y,z) = (t1,t2,n)
 }
 
-// v.v, B.B and v.B of the left (SIDE 0) and right (SIDE 1) state of a face.  The FP32 form may
-// contract multiply-adds.  In the pencil walks (WALK = the reconstruction option, 0 in the lane
-// sweeps) it names the products that it contracts, so that the rounding of a face does not follow
-// the code around it.
+// v.v, B.B and v.B of the left (SIDE 0) and right (SIDE 1) state of a face.  The FP32 form may contract
+// multiply-adds, and of a sum of products the compiler contracts one or another by the code around it.  In
+// the pencil walks (WALK = the reconstruction option, 0 in the lane sweeps) the contracted products are
+// named.  Which they are has no reason in the sum: they are the ones that were contracted while every cell
+// formed both its face values, per sweep, side and (first limiter against the others) reconstruction, so that
+// sharing the face values changed no bit of a flux.  They hold for LF and HLL behind PPM and TVD and for HLLC
+// behind PPM, each compared flux for flux; the other forms take the walk that names nothing (flux_walk_plain).
 template <int DIR, int SIDE, int WALK, typename R>
 __host__ __device__ inline R vsq_side(R vn, R vt1, R vt2)
 {
@@ -662,12 +665,12 @@ __host__ __device__ inline void lf_face(R g, const FaceState<R> &L, const FaceSt
 // outer speeds min/max(v_nL, v_nR) -/+ max(c_fL, c_fR) (eq. 67); contact speed S_M and p_T*
 // (eqs. 38, 41); single-star states (eqs. 43-48, degenerate denominators keep the transverse v
 // and B); Alfven speeds S_M -/+ |B_n|/sqrt(rho*) (eq. 51); double-star states (eqs. 59-63).
-template <int DIR, typename R, int WALK = 0>
+template <int DIR, typename R>
 __host__ __device__ inline void hlld_face(R g, const FaceState<R> &L, const FaceState<R> &Rr, R f[7])
 {
     Side7<R> s[2];
-    face_side<DIR, 0, WALK, R>(g, L, s[0]);
-    face_side<DIR, 1, WALK, R>(g, Rr, s[1]);
+    face_side<DIR, 0, 0, R>(g, L, s[0]);
+    face_side<DIR, 1, 0, R>(g, Rr, s[1]);
     const R bn = L.bn;
     const R cmax = fmax2<R>(s[0].cf, s[1].cf);
     const R sL = fmin2<R>(s[0].vn, s[1].vn) - cmax;
@@ -817,7 +820,7 @@ __host__ __device__ inline void riemann_face(R g, const FaceState<R> &L, const F
 {
     if (SOLVER == 1) lf_face<DIR, R, WALK>(g, L, Rr, f);
     else if (SOLVER == 3) hllc_face<DIR, R, WALK>(g, L, Rr, f);
-    else if (SOLVER == 4) hlld_face<DIR, R, WALK>(g, L, Rr, f);
+    else if (SOLVER == 4) hlld_face<DIR, R>(g, L, Rr, f);
     else hll_face<DIR, R, WALK>(g, L, Rr, f);
 }
 
