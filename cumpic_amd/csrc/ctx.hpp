@@ -246,6 +246,17 @@ static inline bool y_lanes(const Lay &L, int seg)
 {
     return L.ny >= 16 && (long)L.px * flux_planes(L) * nblk(L.ny + 1, seg) < YLANE_WALKERS;
 }
+// An FP64 grid of a few long pencils along y (a 1D problem laid along y, a strip): the lanes of a walk's
+// wavefront are pencils, so at most 12 of 64 would work, while a wavefront of the wave-parallel form takes 59
+// faces of one.  That form is a launch of its own, which short pencils do not earn.  Per step, walks in the
+// joined launch against the wave-parallel sweep beside it: 1 x 2000 cells 110 / 116 us, 1 x 5000 151 / 132,
+// 1 x 100000 983 / 723, 10 x 5000 171 / 164, 10 x 100000 1538 / 1422, 18 x 100000 2317 / 2352; three planes
+// 1 x 20000 x 1 666 / 669, 1 x 50000 x 1 1947 / 1830.
+static inline bool thin_y(const Lay &L)
+{
+    const int npl = flux_planes(L);
+    return (L.nx + 2) * npl <= 12 && L.ny >= 4096 * npl;
+}
 // What the tuned segment length comes to in the y and z sweeps of a run: values that come to the same are one
 // launch shape, which the tuner times once.
 static inline std::array<int, 3> seg_shape(const Lay &L, bool mixed, int seg)
@@ -276,6 +287,12 @@ void launch_fluxes_t(cumc_ctx *ctx, const Lay &L, const Fields<R> &F, int only_d
             G.z_n = G.z_gx * nz;
             G.x_waves = (int)xw;
             mark(ctx, KC_FLUX_XYZ);
+            if (thin_y(L)) {
+                const int gx = ylane_groups(L) * ylane_segs(L);
+                hipLaunchKernelGGL((k_flux_ylane<R, RECON, SOLVER>), dim3(xcd_blocks(gx, npl)), dim3(256), 0, s, L, F, tb, M,
+                                   gx, npl);
+                G.y_n = 0;
+            }
             hipLaunchKernelGGL((k_flux_xyz<RECON, SOLVER>), dim3((unsigned)(G.y_n + G.z_n + xw * npl)), dim3(64), 0, s, L, F,
                                tb, M, G);
             mark(ctx, -1);

@@ -242,11 +242,12 @@ __global__ __launch_bounds__(256) void k_flux_x(Lay L, Fields<R> F, Tabs tb, Mod
 // leave most of the GPU idle), wave-parallel like the x sweep: a wavefront holds 64 consecutive
 // cells of one y pencil, neighbours by lane moves, and emits its 59 faces; the four wavefronts
 // of a workgroup take neighbouring pencils j, so the rows they load (stride px) meet in the same
-// 128-byte lines.  The same reconstruction and Riemann solve as the pencil walk, bit for bit.
+// 128-byte lines.  The same reconstruction and Riemann solve as the pencil walk: in FP64 bit for bit, in
+// FP32 but for which product of a sum is contracted.
 // Tile bx of plane l: 4-pencil group bx % njt (j in [0, nx+1]) of segment bx / njt.
 // The mixed form takes it where its walks in segments of the tuned length would run fewer than
 // YLANE_WALKERS threads (one wavefront per SIMD of the 256 CUs); the FP64 sweeps run in one launch
-// (k_flux_xyz), whose short walks are the faster ones.
+// (k_flux_xyz), whose short walks are the faster ones but for a few long pencils (thin_y).
 // ------------------------------------------------------------------------------------------
 constexpr long YLANE_WALKERS = 1024L * 64;
 __host__ __device__ inline int ylane_groups(const Lay &L) { return (L.nx + 2 + 3) / 4; }

@@ -105,3 +105,33 @@ def test_one_launch_matches_separate_sweeps(grid):
         g.close()
     for k in ("prim", "eps", "bcell"):
         assert_bitwise(states[0][k], states[1][k], k)
+
+
+# a few long pencils along y: the wave-parallel y sweep beside the joined one, and grids just short of it;
+# one plane (z-collapsed) and the three planes of a box that is not
+@pytest.mark.parametrize("recon", [4, 1])
+@pytest.mark.parametrize("nx,ny,collapse", [(1, 4096, True), (2, 4200, True), (10, 4160, True), (11, 4160, True), (1, 4095, True),
+                                            (2, 12288, False), (3, 12288, False)])
+def test_long_thin_grids_match_restatement(nx, ny, collapse, recon):
+    from cumpic_amd.config import Config, uniform_faces
+    from cumpic_amd.cumc import Solver
+    from cumpic_amd.ics import Problem
+    from oracle.oracle import Oracle
+    cfg = Config(nx=nx, ny=ny, nz=1, boundary_flag=(1,) * 6, recon=recon, cfl=0.3)
+    rng = np.random.default_rng(7)
+    prim = rng.uniform(-0.2, 0.2, cfg.shape + (8,))
+    prim[..., 0], prim[..., 4] = rng.uniform(0.5, 1.5, cfg.shape), rng.uniform(0.5, 1.5, cfg.shape)
+    prob = Problem(cfg, uniform_faces(nx, 0.0, 1.0), uniform_faces(ny, 0.0, 64.0), uniform_faces(1, 0.0, 1.0), prim,
+                   prim[..., 4] / prim[..., 0] / (cfg.ggas - 1.0))
+    g, o = Solver.from_problem(prob), Oracle.from_problem(prob)
+    g.set_zcollapse(collapse)
+    g.initial_update()
+    o.initial_update()
+    for _ in range(2):
+        dt = g.finddt()
+        assert dt == o.finddt()
+        g.rungekutta(dt)
+        o.rungekutta(dt)
+    a, b = g.download(), o.get_state()
+    for k in ("prim", "eps", "bcell"):
+        assert_bitwise(a[k], b[k], k)
