@@ -16,9 +16,10 @@ namespace {
 constexpr size_t UNIT_BYTES = size_t(2) << 20;  // of device memory and of pinned host memory, per unit
 constexpr int MAX_UNITS = 8;                    // per device: at most 16 MiB of either kind of memory
 constexpr int MAX_DEVICES = 64;
-// A transfer takes one more unit per this much.  Below it a second thread costs more than it saves: download of
-// 22^3 (2.1 MB) 144 us on one, 164 on two; of 36^3 267 on two, 312 on three.
-constexpr size_t BYTES_PER_UNIT = size_t(3) << 20;
+// A transfer takes one more unit per this much: less for downloads, whose threads also take the page faults of the
+// caller's fresh array.  One thread against two: download of 22^3 (2.6 MB) 143 / 119 us, upload of 24^3 (1.9 MB)
+// 121 / 124; two against three: download of 30^3 (5.4 MB) 243 / 186.
+constexpr size_t BYTES_PER_UNIT_IN = size_t(2) << 20, BYTES_PER_UNIT_OUT = size_t(3) << 19;
 // A stream costs about 0.75 ms to make and destroy, in which one unit moves about this much.
 constexpr double STREAM_BYTES = double(4 << 20);
 
@@ -35,7 +36,7 @@ struct Block {
 };
 struct Device {
     int units = 0, streams = 0;  // made, idle or in use
-    double owed = 0.0;           // bytes' worth of time that one more stream would have saved so far
+    int transfers = 0;           // since the first context
     std::vector<hipStream_t> idle;
 };
 
@@ -86,11 +87,10 @@ struct Lease {
     // At least one unit of the current device and at most `want`, for a transfer of `bytes`.  A call waits
     // only while other transfers hold all of them; none are held while waiting, so every waiter is served
     // in the end.  No units: out of memory.
-    // One more unit at a time is worth a stream once the time it saves, here or added up over the transfers
-    // so far, is the time the stream takes to make and destroy: a process that opens a context, moves little
-    // and closes it again must not pay for eight.  64^3 opened, uploaded, stepped four times, downloaded and
-    // closed: 15.5 ms with eight units made one by one at the first transfer, 5.5 ms so; repeated transfers
-    // have as many units as before after the first few.
+    // The first two transfers (a state up, a result down) take one more unit only while that saves them more
+    // than its stream costs: a process that opens a context, moves little and closes it again must not pay for
+    // eight.  From the third on a transfer takes all it can use.  64^3 opened, uploaded, stepped four times,
+    // downloaded and closed: 15.5 ms with eight units made one by one at the first transfer, 6.4 ms so.
     void take(int dev, int want, double bytes)
     {
         device = dev;
@@ -99,6 +99,7 @@ struct Lease {
         streams.reserve(want);
         std::unique_lock<std::mutex> lock(g_mu);
         d.idle.reserve(MAX_UNITS);
+        d.transfers++;
         for (;;) {
             int free = 0;
             for (const Unit &u : g_free) free += u.device == dev;
@@ -123,14 +124,12 @@ struct Lease {
                 d.idle.pop_back();
             } else {
                 const double k = (double)streams.size() + 1.0;
-                d.owed += bytes / (k * (k + 1.0));
-                if (d.streams >= MAX_UNITS - 1 || d.owed < STREAM_BYTES) break;
+                if (d.streams >= MAX_UNITS - 1 || (d.transfers <= 2 && bytes / (k * (k + 1.0)) < STREAM_BYTES)) break;
                 if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
                     (void)hipGetLastError();
                     break;
                 }
                 d.streams++;
-                d.owed = 0.0;
             }
             streams.push_back(s);
         }
@@ -189,12 +188,13 @@ struct Piece {
     int n;
 };
 
-// One thread's pieces through one unit and one stream.  They are queued until the unit is full and waited
-// for together, conversions next to each other and copies next to each other (going from one engine to the
-// other and back costs about 15 us): a box that fits into a unit costs one wait.
+// One thread's pieces through one unit and one stream.  A thread alone queues them until the unit is full and
+// waits for them together, conversions next to each other and copies next to each other (going from one engine to
+// the other and back costs about 15 us): a box that fits into a unit costs one wait.  Of several threads each waits
+// for every piece, so that one does not queue what another could start.
 struct Worker {
     const Lay &L;
-    bool out;
+    bool out, alone;
     const Unit &u;
     hipStream_t st;
     size_t used = 0;  // bytes of the unit that queued pieces hold
@@ -241,7 +241,7 @@ struct Worker {
         }
         queued.emplace_back(&p, off);
         used += (bytes + 255) / 256 * 256 < UNIT_BYTES - used ? (bytes + 255) / 256 * 256 : UNIT_BYTES - used;
-        return e;
+        return e == hipSuccess && !alone ? flush() : e;
     }
     // shares the pieces with the other workers; leaves nothing queued, after an error either (the unit goes
     // back for the next transfer to use)
@@ -267,15 +267,27 @@ int transfer(cumc_ctx *ctx, const XferArray *a, int n, bool out)
     try {
         size_t bytes = 0;
         for (int i = 0; i < n; i++) bytes += (size_t)ncell * a[i].nv * sizeof(double);
-        const int want = bytes / BYTES_PER_UNIT + 1 > MAX_UNITS ? MAX_UNITS : (int)(bytes / BYTES_PER_UNIT + 1);
+        const size_t per_unit = out ? BYTES_PER_UNIT_OUT : BYTES_PER_UNIT_IN;
+        const int want = bytes / per_unit + 1 > MAX_UNITS ? MAX_UNITS : (int)(bytes / per_unit + 1);
         Lease lease;
         lease.take(device, want, (double)bytes);
         if (lease.units.empty()) return fail(ctx, CUMC_ENOMEM, "transfer staging");
-        // pieces of at most a unit for several threads, of equal size and as many for one as for another; of a
-        // third of a unit for one thread, so that copying one overlaps the engine's work on the one before
-        const size_t k = lease.units.size(), rounds = bytes / (k * UNIT_BYTES) + 1;
-        const size_t share = k > 1 ? bytes / (k * rounds) + 4096 : UNIT_BYTES / 3;
-        const size_t most = share < UNIT_BYTES ? share : UNIT_BYTES;
+        // pieces of at most a unit for several threads, as many for one as for another (the fewest rounds, and the
+        // smallest size that cuts all arrays into no more than that); of a third of a unit for one thread, so that
+        // copying one overlaps the engine's work on the one before
+        const size_t k = lease.units.size();
+        size_t most = UNIT_BYTES / 3;
+        auto cut = [&]() {
+            size_t c = 0;
+            for (int i = 0; i < n; i++) c += ((size_t)ncell * a[i].nv * sizeof(double) + most - 1) / most;
+            return c;
+        };
+        for (size_t rounds = bytes / (k * UNIT_BYTES) + 1; k > 1; rounds++) {
+            most = bytes / (k * rounds);
+            while (most < UNIT_BYTES && cut() > k * rounds) most += most / 64 + 64;
+            most = most < UNIT_BYTES ? most : UNIT_BYTES;
+            if (cut() <= k * rounds) break;
+        }
         std::vector<Piece> pieces;
         for (int i = 0; i < n; i++) {
             const long per = (long)(most / sizeof(double)) / a[i].nv;
@@ -285,7 +297,7 @@ int transfer(cumc_ctx *ctx, const XferArray *a, int n, bool out)
         std::atomic<int> err{(int)hipSuccess};
         std::vector<Worker> workers;
         for (size_t i = 0; i < k; i++) {
-            workers.push_back(Worker{L, out, lease.units[i], i ? lease.streams[i - 1] : ctx->stream});
+            workers.push_back(Worker{L, out, k == 1, lease.units[i], i ? lease.streams[i - 1] : ctx->stream});
             workers[i].queued.reserve(pieces.size());
         }
         std::vector<std::thread> threads;

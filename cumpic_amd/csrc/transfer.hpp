@@ -5,9 +5,9 @@
 // size on each call cost a hipMalloc and hipFree (which waits for the device) and a copy from or to pageable
 // memory at one thread's page-fault rate; here the staging units (2 MiB of either memory) are kept while
 // there is a context, and a large transfer runs up to eight of them at once, one host thread each, so that
-// conversion, copy and the caller's page faults overlap.  Download of 256^3 (1.7 GB) 166 -> 35 ms, of a 400^2
-// box (111 MB, seven planes) 10.0 -> 2.5 ms, of 24^3 200 -> 185 us; upload of 256^3 (1.3 GB) 43 -> 23 ms, of
-// 24^3 122 -> 120 us.
+// conversion, copy and the caller's page faults overlap.  Download of 256^3 (1.7 GB) 166 -> 36 ms, of a 400^2
+// box (111 MB, seven planes) 10.0 -> 2.5 ms, of 24^3 202 -> 157 us; upload of 256^3 (1.3 GB) 43 -> 23 ms, of
+// 24^3 120 -> 119 us.
 #pragma once
 #include "ctx.hpp"
 
