@@ -36,7 +36,7 @@ struct Block {
 };
 struct Device {
     int units = 0, streams = 0;  // made, idle or in use
-    int transfers = 0;           // since the first context
+    int transfers = 0;           // since the first context, counted to three
     std::vector<hipStream_t> idle;
 };
 
@@ -99,7 +99,7 @@ struct Lease {
         streams.reserve(want);
         std::unique_lock<std::mutex> lock(g_mu);
         d.idle.reserve(MAX_UNITS);
-        d.transfers++;
+        if (d.transfers < 3) d.transfers++;
         for (;;) {
             int free = 0;
             for (const Unit &u : g_free) free += u.device == dev;

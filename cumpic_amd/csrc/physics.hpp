@@ -80,7 +80,8 @@ template <> __host__ __device__ inline float sign1(float x) { return copysignf(1
 // numerator is zero or of magnitude in [2^-960, 2^700]; the callers check that (den_ok, num_ok) and
 // take the plain operations for a face where it fails.  (The final correction subtracts the residual,
 // which keeps the sign of a zero numerator.)  root() is sqrt without its scaling and its special
-// cases, for arguments in [2^-700, 2^700].
+// cases, for arguments in [2^-700, 2^700]: Goldschmidt's iteration for the root and half its reciprocal
+// with two residual corrections (Markstein 2004, Proc. RNC6, 146).
 // ------------------------------------------------------------------------------------------
 constexpr double Q_DLO = 0x1p-60, Q_DHI = 0x1p60, Q_NLO = 0x1p-960, Q_NHI = 0x1p700;
 // (the diagnostic build records every decision: it takes the plain form)
@@ -226,8 +227,8 @@ __host__ __device__ inline R ppm_slope(R b0, R b1, R vm1, R vc, R vp1)
 // as the high edge of one cell and the low edge of the next; with the coefficients of ppm_coef
 // (a0p .. a3p of cell j equal a0m .. a3m of cell j+1, expression by expression) both are this value
 // bit for bit, so the sweeps form it once per face: 16 to 17 operations and a lane move less per
-// variable and cell with the shared differences and the min instructions (x sweep 1264 -> 1147 VALU
-// instructions, y walk 1482 -> 1276; 128^3 FP64 2.62 -> 2.36 ms per step).
+// variable and cell with the shared differences and the min instructions (compiled x sweep 1264 -> 1147
+// VALU instructions, y walk 1482 -> 1276; 128^3 FP64 2.62 -> 2.36 ms per step).
 template <typename R>
 __host__ __device__ inline R ppm_face(R a0, R a1, R a2, R a3, R vc, R d, R dm_hi, R dm_lo)
 {

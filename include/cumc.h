@@ -140,7 +140,8 @@ const char *cumc_last_error(cumc_ctx *ctx);
 
 /* ------------------------------------------------------------------------------------------
  * Launch-shape tuning.  No reference counterpart (OpenACC picks gangs/vectors itself); the
- * shapes change no result bit.
+ * shapes change no result bit, but in the mixed form seg can choose the other y sweep of a small
+ * grid, whose FP32 fluxes differ in the last bit.
  * ------------------------------------------------------------------------------------------ */
 enum { CUMC_PH_FLUX_X = 0, CUMC_PH_FLUX_Y, CUMC_PH_FLUX_Z, CUMC_PH_ECORN, CUMC_PH_TAIL, CUMC_PH_GHOST,
        CUMC_PH_FINDDT, CUMC_PH_N };
